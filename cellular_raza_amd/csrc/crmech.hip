@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <charconv>
 #include <cmath>
 #include <cstdio>
@@ -162,6 +163,25 @@ static void fill_pot(PotParams<T>& q, const crm_potential& p) {
 
 enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 
+// ---- host transfers ---------------------------------------------------------
+// Each context owns a pinned block: the control block's copy, then kPinWorkers
+// chunks of kPinChunkSmall bytes.  Read-backs of small systems are written there by
+// the gathering kernel; larger ones are copied out chunk by chunk, each chunk emptied
+// by a host thread of its own: one thread fills fresh pages of the caller's array at
+// 4.5 GB/s (page faults), two at 8, four at 12.5, eight at 19-20 GB/s (48 MB and
+// 192 MB; the link carries 55 GB/s).  Read-backs above kPinLarge get kPinChunkLarge
+// chunks, allocated on the first one (48 MB: 2.7 ms in either size, 192 MB: 9.9 ms
+// against 10.9 with half of it); an allocation takes 0.1 ms up to 2 MB, 0.3 ms at 8.
+constexpr size_t kPinControl = 4096;
+constexpr uint32_t kPinWorkers = 8;
+constexpr size_t kPinChunkSmall = 256 * 1024;
+constexpr size_t kPinChunkLarge = 1024 * 1024;
+constexpr size_t kPinLarge = 8 * 1024 * 1024;
+// Largest read-back that the kernel writes to pinned memory itself: get_state takes
+// 36 us at 259 KB, and 94 us at 269 KB through two host threads (256 KB and more to a
+// thread is where a second one pays for its start).
+constexpr size_t kPinDirect = 256 * 1024;
+
 // ---- device scratch of crm_remove_agents_noalloc ---------------------------
 // One static array per GPU, sized for kNoAllocMaxAgents agents in at most
 // kNoAllocMaxInstances instances: flags [n] bytes, four [n + 1] uint32 arrays
@@ -285,6 +305,10 @@ struct crm_ctx {
     int t_used = 0;
     double t_ms[CRM_KERNEL_COUNT] = {};
     uint64_t t_n[CRM_KERNEL_COUNT] = {};
+
+    uint8_t* pin = nullptr;        // kPinControl bytes + kPinWorkers chunks of kPinChunkSmall
+    uint8_t* pin_large = nullptr;  // kPinWorkers chunks of kPinChunkLarge
+    hipEvent_t pin_ev[kPinWorkers] = {};
 };
 
 namespace {
@@ -760,16 +784,23 @@ crm_status launch_step(crm_ctx* ctx, const double* noise_step) {
     return CRM_OK;
 }
 
+// The control block after everything queued so far: a one-thread kernel writes it
+// to the context's pinned page (launch and wait 11 us; a copy to pageable memory 24).
 crm_status read_control(crm_ctx* ctx, Control& c) {
-    CRM_HIP(hipMemcpyAsync(&c, ctx->d_ctrl, sizeof(Control), hipMemcpyDeviceToHost, ctx->stream));
+    hipLaunchKernelGGL(k_publish_control, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl,
+                       reinterpret_cast<Control*>(ctx->pin));
+    CRM_HIP(hipGetLastError());
     CRM_HIP(hipStreamSynchronize(ctx->stream));
+    std::memcpy(&c, ctx->pin, sizeof(Control));
     return CRM_OK;
 }
 
-// Maps the device error word to a status and message.
-crm_status check_errors(crm_ctx* ctx, const char* phase) {
+// Maps the device error word to a status and message (`known`: the control block
+// when the caller has just read it).
+crm_status check_errors(crm_ctx* ctx, const char* phase, const Control* known = nullptr) {
     Control c;
-    CRM_TRY(read_control(ctx, c));
+    if (known) c = *known;
+    else CRM_TRY(read_control(ctx, c));
     if (!c.error_flags) return CRM_OK;
     crm_status kind = CRM_CALC_ERROR;
     const char* msg = "CalcError: identical position for two objects. Cannot Calculate force in Mie potential";
@@ -902,14 +933,105 @@ crm_status upload_tiles(crm_ctx* ctx, const std::vector<ForceTile>& tiles) {
     return CRM_OK;
 }
 
-// Downloads a [C][N] SoA array and reorders it to agent index (rows of C).
-crm_status download_by_id(crm_ctx* ctx, const double* d_src, uint32_t C, double* out,
-                          const std::vector<uint32_t>& id) {
-    std::vector<double> tmp((size_t)C * ctx->N);
-    CRM_HIP(hipMemcpyAsync(tmp.data(), d_src, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+// One device range and the host memory it goes to.
+struct HostPiece {
+    const uint8_t* dev;
+    uint8_t* host;
+    size_t bytes;
+};
+
+// Copies the pieces to pageable host memory, chunk by chunk through pinned memory:
+// every host thread takes the next chunk, queues its copy into its own pinned chunk
+// and moves it on once it has arrived.  The stream's earlier work precedes the copies.
+crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
+    size_t total = 0;
+    for (int i = 0; i < n_pieces; i++) total += pieces[i].bytes;
+    const bool large = total > kPinLarge;
+    if (large && !ctx->pin_large)
+        CRM_HIP(hipHostMalloc((void**)&ctx->pin_large, kPinWorkers * kPinChunkLarge, hipHostMallocDefault));
+    uint8_t* const pins = large ? ctx->pin_large : ctx->pin + kPinControl;
+    const size_t chunk = large ? kPinChunkLarge : kPinChunkSmall;
+    size_t n_chunks = 0;
+    for (int i = 0; i < n_pieces; i++) n_chunks += (pieces[i].bytes + chunk - 1) / chunk;
+    const uint32_t hw = std::max(1u, std::thread::hardware_concurrency() / 2);
+    const uint32_t workers = (uint32_t)std::min<size_t>(std::min(kPinWorkers, hw), std::max<size_t>(n_chunks, 1));
+    for (uint32_t w = 0; w < workers; w++)
+        if (!ctx->pin_ev[w]) CRM_HIP(hipEventCreateWithFlags(&ctx->pin_ev[w], hipEventDisableTiming));
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&](uint32_t w) {
+        hipError_t e = hipSetDevice(ctx->device);
+        uint8_t* const pin = pins + w * chunk;
+        while (e == hipSuccess && failed.load() == (int)hipSuccess) {
+            size_t c = next.fetch_add(1);
+            int i = 0;
+            for (; i < n_pieces; i++) {
+                const size_t nc = (pieces[i].bytes + chunk - 1) / chunk;
+                if (c < nc) break;
+                c -= nc;
+            }
+            if (i == n_pieces) return;
+            const size_t off = c * chunk, len = std::min(chunk, pieces[i].bytes - off);
+            e = hipMemcpyAsync(pin, pieces[i].dev + off, len, hipMemcpyDeviceToHost, ctx->stream);
+            if (e == hipSuccess) e = hipEventRecord(ctx->pin_ev[w], ctx->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(ctx->pin_ev[w]);
+            if (e == hipSuccess) std::memcpy(pieces[i].host + off, pin, len);
+        }
+        if (e != hipSuccess) failed.store((int)e);
+    };
+    std::thread threads[kPinWorkers];
+    for (uint32_t w = 1; w < workers; w++) {
+        try {
+            threads[w] = std::thread(work, w);
+        } catch (...) {  // no more threads to be had: the ones running share the chunks
+            break;
+        }
+    }
+    work(0);
+    for (auto& t : threads)
+        if (t.joinable()) t.join();
+    CRM_HIP((hipError_t)failed.load());
+    return CRM_OK;
+}
+
+// A [C][N] array by slot (double, or the mixed path's float forces) to be read as
+// rows of C by agent index.
+struct RowRead {
+    const void* src;
+    bool f32;
+    uint32_t C;
+    double* out;
+};
+
+// Reads up to two arrays.  The rows are gathered on the device, for small systems
+// straight into pinned host memory, else into the other state buffer (free between
+// steps: every step writes it whole before it reads it) and copied out from there.
+crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n) {
+    const uint64_t N = ctx->N;
+    size_t total = 0;
+    for (int i = 0; i < n; i++) total += (size_t)N * r[i].C * sizeof(double);
+    const bool small = total <= kPinDirect;
+    double* scratch[2] = {ctx->buf[1 - ctx->cur].pos, ctx->buf[1 - ctx->cur].vel};
+    HostPiece piece[2];
+    uint8_t* pin = ctx->pin + kPinControl;
+    for (int i = 0; i < n; i++) {
+        const size_t bytes = (size_t)N * r[i].C * sizeof(double);
+        double* dst = small ? reinterpret_cast<double*>(pin) : scratch[i];
+        piece[i] = HostPiece{reinterpret_cast<const uint8_t*>(dst), reinterpret_cast<uint8_t*>(r[i].out), bytes};
+        pin += bytes;
+        const dim3 g((uint32_t)((N + kBlock - 1) / kBlock)), b(kBlock);
+        const uint32_t* id = ctx->buf[ctx->cur].id;
+        if (r[i].f32)
+            hipLaunchKernelGGL(k_rows_by_id<float>, g, b, 0, ctx->stream, static_cast<const float*>(r[i].src), id, dst,
+                               N, r[i].C);
+        else
+            hipLaunchKernelGGL(k_rows_by_id<double>, g, b, 0, ctx->stream, static_cast<const double*>(r[i].src), id,
+                               dst, N, r[i].C);
+        CRM_HIP(hipGetLastError());
+    }
+    if (!small) return copy_out(ctx, piece, n);
     CRM_HIP(hipStreamSynchronize(ctx->stream));
-    for (uint64_t s = 0; s < ctx->N; s++)
-        for (uint32_t k = 0; k < C; k++) out[(uint64_t)id[s] * C + k] = tmp[(uint64_t)k * ctx->N + s];
+    for (int i = 0; i < n; i++) std::memcpy(piece[i].host, piece[i].dev, piece[i].bytes);
     return CRM_OK;
 }
 
@@ -1801,6 +1923,8 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
     if (hipMalloc((void**)&ctx->d_ip, sizeof(InstParams) * n_instances) != hipSuccess ||
         hipMalloc((void**)&ctx->d_ctrl, sizeof(Control)) != hipSuccess)
         return fail(CRM_DEVICE_ERROR, "hipMalloc failed");
+    if (hipHostMalloc((void**)&ctx->pin, kPinControl + kPinWorkers * kPinChunkSmall, hipHostMallocDefault) != hipSuccess)
+        return fail(CRM_DEVICE_ERROR, "hipHostMalloc failed");
     e = hipMemcpy(ctx->d_ip, ctx->hparams.data(), sizeof(InstParams) * n_instances, hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipMemcpy: ") + hipGetErrorString(e));
     *out = ctx;
@@ -1921,22 +2045,20 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
     ctx->cur = 0;
     StateBuf& S = ctx->buf[0];
     {
-        std::vector<double> tp((size_t)K * N), tv((size_t)K * N, 0.0);
-        for (uint64_t a = 0; a < N; a++)
-            for (uint32_t k = 0; k < K; k++) {
-                tp[(uint64_t)k * N + a] = pos[a * K + k];
-                if (vel) tv[(uint64_t)k * N + a] = vel[a * K + k];
-            }
-        std::vector<int32_t> sp(N, 0);
-        std::vector<uint32_t> id(N);
-        for (uint64_t a = 0; a < N; a++) {
-            sp[a] = species ? species[a] : 0;
-            id[a] = (uint32_t)a;
+        // rows into the other buffer, put in slot order by a kernel
+        const dim3 g((uint32_t)((N + kBlock - 1) / kBlock)), b(kBlock);
+        double* rows = ctx->buf[1].pos;
+        CRM_HIP(hipMemcpyAsync(rows, pos, (size_t)K * N * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+        hipLaunchKernelGGL(k_rows_to_slots, g, b, 0, ctx->stream, rows, S.pos, N, K);
+        if (vel) {
+            rows = ctx->buf[1].vel;
+            CRM_HIP(hipMemcpyAsync(rows, vel, (size_t)K * N * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
         }
-        CRM_HIP(hipMemcpyAsync(S.pos, tp.data(), tp.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-        CRM_HIP(hipMemcpyAsync(S.vel, tv.data(), tv.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-        CRM_HIP(hipMemcpyAsync(S.species, sp.data(), N * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-        CRM_HIP(hipMemcpyAsync(S.id, id.data(), N * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+        hipLaunchKernelGGL(k_rows_to_slots, g, b, 0, ctx->stream, vel ? rows : nullptr, S.vel, N, K);
+        if (species)
+            CRM_HIP(hipMemcpyAsync(S.species, species, N * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+        hipLaunchKernelGGL(k_initial_ids, g, b, 0, ctx->stream, species ? nullptr : S.species, S.id, N);
+        CRM_HIP(hipGetLastError());
         if (is_rod(ctx)) {
             // per-rod spring length from the instance, first push at step 0,
             // growth at the cycle's base rate, CellIdentifier::Initial(index in
@@ -2069,7 +2191,7 @@ crm_status crm_step(crm_ctx* ctx, uint32_t n_steps, const double* noise) {
     ctx->step += done;
     // the last step's forces (and counts) read the buffer before its gather
     if (done > 0) ctx->sense_parity = 1 - ctx->cur;
-    return check_errors(ctx, "step");
+    return check_errors(ctx, "step", &c);
 }
 
 crm_status crm_compute_forces(crm_ctx* ctx, double* force) {
@@ -2077,28 +2199,20 @@ crm_status crm_compute_forces(crm_ctx* ctx, double* force) {
     if (!ctx->have_agents) return CRM_INVALID_ARGUMENT;
     CRM_HIP(hipSetDevice(ctx->device));
     CRM_TRY(launch_force(ctx));
-    CRM_HIP(hipStreamSynchronize(ctx->stream));
-    crm_status st = check_errors(ctx, "forces");
-    if (st) return st;
-    std::vector<uint32_t> id;
-    CRM_TRY(download_ids(ctx, id));
-    if (!force_f32(ctx)) return download_by_id(ctx, ctx->d_force, ctx->K, force, id);
-    std::vector<float> tmp((size_t)ctx->K * ctx->N);
-    CRM_HIP(hipMemcpyAsync(tmp.data(), ctx->d_force, tmp.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    CRM_HIP(hipStreamSynchronize(ctx->stream));
-    for (uint64_t s = 0; s < ctx->N; s++)
-        for (uint32_t k = 0; k < ctx->K; k++) force[(uint64_t)id[s] * ctx->K + k] = (double)tmp[(uint64_t)k * ctx->N + s];
-    return CRM_OK;
+    CRM_TRY(check_errors(ctx, "forces"));
+    const RowRead r{ctx->d_force, force_f32(ctx), ctx->K, force};
+    return read_rows(ctx, &r, 1);
 }
 
 crm_status crm_get_state(crm_ctx* ctx, double* pos, double* vel) {
     if (!ctx || !ctx->have_agents) return CRM_INVALID_ARGUMENT;
     CRM_HIP(hipSetDevice(ctx->device));
-    std::vector<uint32_t> id;
-    CRM_TRY(download_ids(ctx, id));
-    if (pos) CRM_TRY(download_by_id(ctx, ctx->buf[ctx->cur].pos, ctx->K, pos, id));
-    if (vel) CRM_TRY(download_by_id(ctx, ctx->buf[ctx->cur].vel, ctx->K, vel, id));
-    return CRM_OK;
+    const StateBuf& S = ctx->buf[ctx->cur];
+    RowRead r[2];
+    int n = 0;
+    if (pos) r[n++] = RowRead{S.pos, false, ctx->K, pos};
+    if (vel) r[n++] = RowRead{S.vel, false, ctx->K, vel};
+    return n ? read_rows(ctx, r, n) : CRM_OK;
 }
 
 crm_status crm_get_history(crm_ctx* ctx, double* dx_hist, double* dv_hist, uint32_t* n_stored) {
@@ -2109,10 +2223,10 @@ crm_status crm_get_history(crm_ctx* ctx, double* dx_hist, double* dv_hist, uint3
     const uint32_t size = cap == 0 ? 0u : (uint32_t)std::min<uint64_t>(t, cap);
     const uint32_t oldest = (size < cap || cap == 0) ? 0u : (uint32_t)(t % cap);
     if (n_stored) *n_stored = size;
-    std::vector<uint32_t> id;
-    CRM_TRY(download_ids(ctx, id));
     const uint64_t slot_elems = (uint64_t)ctx->N * ctx->K;
     if (ctx->pt_births) {  // inserted agents hold the pushes since their birth, oldest first, then zeros
+        std::vector<uint32_t> id;
+        CRM_TRY(download_ids(ctx, id));
         const uint64_t N = ctx->N;
         const uint32_t K = ctx->K;
         std::vector<double> hx(2 * slot_elems), hv(2 * slot_elems);
@@ -2143,12 +2257,12 @@ crm_status crm_get_history(crm_ctx* ctx, double* dx_hist, double* dv_hist, uint3
     for (uint32_t i = 0; i < 2; i++) {
         if (i < size) {
             uint32_t slot = (oldest + i) % cap;
-            if (dx_hist)
-                CRM_TRY(download_by_id(ctx, ctx->buf[ctx->cur].hdx + slot * slot_elems, ctx->K,
-                                       dx_hist + i * slot_elems, id));
-            if (dv_hist)
-                CRM_TRY(download_by_id(ctx, ctx->buf[ctx->cur].hdv + slot * slot_elems, ctx->K,
-                                       dv_hist + i * slot_elems, id));
+            RowRead r[2];
+            int n = 0;
+            const StateBuf& S = ctx->buf[ctx->cur];
+            if (dx_hist) r[n++] = RowRead{S.hdx + slot * slot_elems, false, ctx->K, dx_hist + i * slot_elems};
+            if (dv_hist) r[n++] = RowRead{S.hdv + slot * slot_elems, false, ctx->K, dv_hist + i * slot_elems};
+            if (n) CRM_TRY(read_rows(ctx, r, n));
         } else {
             if (dx_hist) std::fill(dx_hist + i * slot_elems, dx_hist + (i + 1) * slot_elems, 0.0);
             if (dv_hist) std::fill(dv_hist + i * slot_elems, dv_hist + (i + 1) * slot_elems, 0.0);
@@ -2384,8 +2498,14 @@ crm_status crm_get_cycle_state(crm_ctx* ctx, double* spring_length, double* grow
     CRM_TRY(download_ids(ctx, id));
     const uint64_t N = ctx->N;
     const StateBuf& S = ctx->buf[ctx->cur];
-    if (spring_length) CRM_TRY(download_by_id(ctx, S.spring, 1, spring_length, id));
-    if (growth_rate) CRM_TRY(download_by_id(ctx, S.growth, 1, growth_rate, id));
+    if (spring_length) {
+        const RowRead r{S.spring, false, 1, spring_length};
+        CRM_TRY(read_rows(ctx, &r, 1));
+    }
+    if (growth_rate) {
+        const RowRead r{S.growth, false, 1, growth_rate};
+        CRM_TRY(read_rows(ctx, &r, 1));
+    }
     std::vector<uint64_t> tmp(3 * N);
     uint64_t* outs[2] = {identifier, parent};
     uint64_t* srcs[2] = {S.ident, S.parent};
@@ -2741,6 +2861,10 @@ void crm_destroy(crm_ctx* ctx) {
     free_device(ctx);
     if (ctx->d_ip) (void)hipFree(ctx->d_ip);
     if (ctx->d_ctrl) (void)hipFree(ctx->d_ctrl);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
+    if (ctx->pin_large) (void)hipHostFree(ctx->pin_large);
+    for (auto e : ctx->pin_ev)
+        if (e) (void)hipEventDestroy(e);
     for (int i = 0; i < crm_ctx::kTimingPairs; i++) {
         if (ctx->ev_a[i]) (void)hipEventDestroy(ctx->ev_a[i]);
         if (ctx->ev_b[i]) (void)hipEventDestroy(ctx->ev_b[i]);

@@ -59,4 +59,35 @@ __global__ __launch_bounds__(kBlock) void k_snapshot(StateBuf S, SnapshotArgs a)
     }
 }
 
+// Rows by agent index from a [C][N] array by slot.  Thread per slot: the reads of a
+// component are coalesced, a thread's row is written by consecutive stores that
+// merge in L2.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_rows_by_id(const T* __restrict__ src, const uint32_t* __restrict__ id,
+                                                        double* __restrict__ out, uint64_t N, uint32_t C) {
+    const uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (s >= N) return;
+    double* o = out + (uint64_t)id[s] * C;
+    for (uint32_t k = 0; k < C; k++) o[k] = (double)src[(uint64_t)k * N + s];
+}
+
+// Rows [N][C] by agent index -> [C][N] by slot with slot = agent index (zeros
+// without rows): the state before the first sort.
+__global__ __launch_bounds__(kBlock) void k_rows_to_slots(const double* __restrict__ rows, double* __restrict__ out,
+                                                           uint64_t N, uint32_t C) {
+    const uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (s >= N) return;
+    for (uint32_t k = 0; k < C; k++) out[(uint64_t)k * N + s] = rows ? rows[s * C + k] : 0.0;
+}
+
+__global__ __launch_bounds__(kBlock) void k_initial_ids(int32_t* __restrict__ species, uint32_t* __restrict__ id,
+                                                         uint64_t N) {
+    const uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (s >= N) return;
+    id[s] = (uint32_t)s;
+    if (species) species[s] = 0;
+}
+
+__global__ void k_publish_control(const Control* ctrl, Control* out) { *out = *ctrl; }
+
 }  // namespace crm

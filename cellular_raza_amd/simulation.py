@@ -261,6 +261,12 @@ class MechanicsBackend:
         self._check(self._lib.crm_get_state(self._h, _dp(pos), _dp(vel)))
         return pos, vel
 
+    def get_positions(self) -> np.ndarray:
+        """The positions of get_state alone."""
+        pos = np.empty((self.n_agents, self.K), dtype=np.float64)
+        self._check(self._lib.crm_get_state(self._h, _dp(pos), None))
+        return pos
+
     def get_history(self):
         dx = np.empty((2, self.n_agents, self.K), dtype=np.float64)
         dv = np.empty((2, self.n_agents, self.K), dtype=np.float64)
@@ -459,7 +465,7 @@ def run_simulation(
                 if mask is not None and np.any(mask):
                     be.remove_agents(mask)
             if access is None:
-                out[it] = be.get_state()[0]
+                out[it] = be.get_positions()
                 continue
             _store_cells(be, access.cells, it, templates)
             access.subdomains.store_single_element(it, 0, sub)
