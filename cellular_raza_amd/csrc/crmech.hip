@@ -151,6 +151,9 @@ static void fill_pot(PotParams<T>& q, const crm_potential& p) {
     q.mie_constant = (T)(p.en / (p.en - p.em) * std::pow(p.en / p.em, p.em / (p.en - p.em)));
     q.mie_en_s = q.en / q.mie_sigma;
     q.mie_em_s = q.em / q.mie_sigma;
+    auto reciprocal = [](T c) { return (T)(c >= (T)1e-18 && c <= (T)1e18 ? (T)1 / c : (T)NAN); };
+    q.inv_two_radius = reciprocal(q.two_radius);
+    q.inv_cutoff = reciprocal(q.cutoff);
     q.epsilon = (T)p.epsilon;
     q.sigma = (T)p.sigma;
     q.rel_range = (T)p.relative_interaction_range;
@@ -213,6 +216,7 @@ struct crm_ctx {
     uint64_t Vt = 0;
     uint32_t pot_kind = 0, mech_kind = 0;
     bool symmetric = true;
+    bool mie_pow = false;  // an instance's Mie exponents are not integers
     std::string err;
 
     int device = 0;
@@ -515,7 +519,9 @@ template <int D>
 crm_status launch_force_d(crm_ctx* ctx, StateBuf S, uint32_t rank) {
     switch (ctx->pot_kind) {
         case CRM_POTENTIAL_MORSE: return launch_force_dp<D, CRM_POTENTIAL_MORSE>(ctx, S, rank);
-        case CRM_POTENTIAL_MIE: return launch_force_dp<D, CRM_POTENTIAL_MIE>(ctx, S, rank);
+        case CRM_POTENTIAL_MIE:
+            return ctx->mie_pow ? launch_force_dp<D, kPotentialMiePow>(ctx, S, rank)
+                                : launch_force_dp<D, CRM_POTENTIAL_MIE>(ctx, S, rank);
         case CRM_POTENTIAL_BOUND_LENNARD_JONES:
             return launch_force_dp<D, CRM_POTENTIAL_BOUND_LENNARD_JONES>(ctx, S, rank);
         case CRM_POTENTIAL_MORSE_SPECIES: return launch_force_dp<D, CRM_POTENTIAL_MORSE_SPECIES>(ctx, S, rank);
@@ -544,8 +550,12 @@ crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S) {
                                phys, no_lds);
             return CRM_OK;
         case CRM_POTENTIAL_MIE:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
-                               no_lds);
+            if (ctx->mie_pow)
+                hipLaunchKernelGGL((k_force_rod<D, kPotentialMiePow, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
+                                   no_lds);
+            else
+                hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
+                                   no_lds);
             return CRM_OK;
         case CRM_POTENTIAL_BOUND_LENNARD_JONES:
             hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_BOUND_LENNARD_JONES, MIXED>), g, b, 0, ctx->stream, A, S,
@@ -1883,6 +1893,7 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
         }
         fill_pot<double>(P.pd, I.potential);
         fill_pot<float>(P.pf, I.potential);
+        if (I.potential.kind == CRM_POTENTIAL_MIE && (P.pd.ien1 < 0 || P.pd.iem1 < 0)) ctx->mie_pow = true;
         const crm_mechanics& M = I.mechanics;
         P.mass = M.mass;
         P.damping = M.damping;

@@ -13,38 +13,11 @@
 namespace crm {
 
 template <typename T>
-__device__ __forceinline__ T dsqrt(T x);
-template <>
-__device__ __forceinline__ double dsqrt<double>(double x) { return sqrt(x); }
-template <>
-__device__ __forceinline__ float dsqrt<float>(float x) { return sqrtf(x); }
-
-template <typename T>
-__device__ __forceinline__ T dexp(T x);
-template <>
-__device__ __forceinline__ double dexp<double>(double x) { return exp(x); }
-template <>
-__device__ __forceinline__ float dexp<float>(float x) { return expf(x); }
-
-template <typename T>
 __device__ __forceinline__ T dpow(T x, T y);
 template <>
 __device__ __forceinline__ double dpow<double>(double x, double y) { return pow(x, y); }
 template <>
 __device__ __forceinline__ float dpow<float>(float x, float y) { return powf(x, y); }
-
-template <typename T>
-__device__ __forceinline__ T dmin(T a, T b);  // Rust f{32,64}::min: NaN-ignoring
-template <>
-__device__ __forceinline__ double dmin<double>(double a, double b) { return fmin(a, b); }
-template <>
-__device__ __forceinline__ float dmin<float>(float a, float b) { return fminf(a, b); }
-template <typename T>
-__device__ __forceinline__ T dmax(T a, T b);
-template <>
-__device__ __forceinline__ double dmax<double>(double a, double b) { return fmax(a, b); }
-template <>
-__device__ __forceinline__ float dmax<float>(float a, float b) { return fmaxf(a, b); }
 
 // x^e for a small non-negative integer e, by binary powering.
 template <typename T>
@@ -59,9 +32,38 @@ __device__ __forceinline__ T ipow(T x, int e) {
     return r;
 }
 
+// ipow(x, e1) and ipow(x, e2) from one chain of squares.
+template <typename T>
+__device__ __forceinline__ void ipow2(T x, int e1, int e2, T& r1, T& r2) {
+    r1 = r2 = T(1);
+    while (e1 | e2) {
+        if (e1 & 1) r1 = r1 * x;
+        if (e2 & 1) r2 = r2 * x;
+        x = x * x;
+        e1 >>= 1;
+        e2 >>= 1;
+    }
+}
+
 template <typename T>
 __device__ __forceinline__ T powe(T x, T e, int ie) {
     return ie >= 0 ? ipow<T>(x, ie) : dpow<T>(x, e);
+}
+
+// A Mie potential whose exponents are not all integers: kernels of its own, so that
+// the common ones hold no pow() (about 200 instructions at each use, and the
+// registers they live in).
+constexpr int kPotentialMiePow = 64;
+
+// (sigma / r)^(en + 1) and (sigma / r)^(em + 1).
+template <bool POW, typename T>
+__device__ __forceinline__ void mie_powers(T sr, const PotParams<T>& P, T& pn, T& pm) {
+    if constexpr (POW) {
+        pn = powe<T>(sr, P.en + T(1), P.ien1);
+        pm = powe<T>(sr, P.em + T(1), P.iem1);
+    } else {
+        ipow2<T>(sr, P.ien1, P.iem1, pn, pm);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -106,27 +108,99 @@ __device__ __forceinline__ void morse_fast(const float* z, float two_radius, flo
     for (int k = 0; k < D; k++) f[k] = z[k] * fi;
 }
 
+// FP64 pair path: one root and one reciprocal serve every quotient of a pair.  The
+// root is Goldschmidt's iteration from v_rsq_f64 with two Newton corrections on the
+// exact residual d2 - g^2, the reciprocal follows from its half inverse by one more
+// residual step, and a quotient z / r is Markstein's z * inv corrected by the exact
+// remainder z - q r: each is the correctly rounded value, as sqrt() and / give it,
+// in 3 operations per quotient where an IEEE division takes 12 (4 of them at a
+// quarter of the rate), and 11 for the root and the reciprocal together: the FP64
+// force kernels are bound by VALU issue, and the 4M-agent Mie lattice's went from 630
+// to 516 us with bitwise the same forces (with the pow() path in its own kernels,
+// which took 48 spilled registers out of this one; with both in one kernel it ran
+// 862 us), the 12,347-rod FP64 step from 124 to 118 us.  `fast` is
+// false outside [2^-900, 2^900] (and for NaN), where the residuals could underflow;
+// such a pair takes sqrt() and /.
+struct RootInv {
+    double r, inv;
+    bool fast;
+};
+__device__ __forceinline__ RootInv root_inv(double d2) {
+    RootInv q;
+    q.fast = d2 >= 0x1p-900 && d2 <= 0x1p900;
+    if (q.fast) {
+        const double y = __builtin_amdgcn_rsq(d2);
+        double g = d2 * y, h = 0.5 * y;
+        const double e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        g = fma(fma(-g, g, d2), h, g);
+        g = fma(fma(-g, g, d2), h, g);
+        q.r = g;
+        const double i = h + h;
+        const double j = fma(i, fma(-g, i, 1.0), i);
+        q.inv = fma(j, fma(-g, j, 1.0), j);
+    } else {
+        q.r = sqrt(d2);
+        q.inv = 1.0 / q.r;
+    }
+    return q;
+}
+
+// a / b from inv = 1 / b (correctly rounded), for a and b far from under- and overflow.
+__device__ __forceinline__ double quotient(double a, double b, double inv) {
+    const double q = a * inv;
+    return fma(fma(-q, b, a), inv, q);
+}
+
+// The same for a parameter a that may be infinite (an interaction without a bound).
+__device__ __forceinline__ double param_over(double a, const RootInv& q) {
+    if (!q.fast) return a / q.r;
+    const double t = quotient(a, q.r, q.inv);
+    return t == t ? t : a * q.inv;
+}
+
+// z / r for the components of a pair's displacement.
+template <int D>
+__device__ __forceinline__ void direction(const double* z, const RootInv& q, double* dir) {
+    if (q.fast) {
+#pragma unroll
+        for (int k = 0; k < D; k++) dir[k] = quotient(z[k], q.r, q.inv);
+    } else {
+#pragma unroll
+        for (int k = 0; k < D; k++) dir[k] = z[k] / q.r;
+    }
+}
+
+// a / c for a parameter c with its reciprocal from the host (NaN where c is no
+// parameter for `quotient`); r in root_inv's fast range.
+__device__ __forceinline__ double over(double a, double c, double inv_c, bool fast) {
+    return fast && inv_c == inv_c ? quotient(a, c, inv_c) : a / c;
+}
+
 // calculate_morse_interaction, interaction.rs:151-182
 template <typename T, int D>
 __device__ __forceinline__ void morse(const T* z, T two_radius, T cutoff, T strength, T stiffness, int cut, T* f) {
     if constexpr (std::is_same<T, float>::value) {
         morse_fast<D>(z, two_radius, cutoff, strength, stiffness, cut, f);
-        return;
+    } else {
+        double d2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
+        const RootInv q = root_inv(d2);
+        const bool beyond = cut < 0 ? (q.r > cutoff) : (cut == 0);
+        if (beyond || q.r == 0.0) {
+#pragma unroll
+            for (int k = 0; k < D; k++) f[k] = 0.0;
+            return;
+        }
+        const double e = exp((-stiffness) * (q.r - two_radius));
+        const double force = (((-2.0 * strength) * stiffness) * e) * (1.0 - e);
+        double dir[D];
+        direction<D>(z, q, dir);
+#pragma unroll
+        for (int k = 0; k < D; k++) f[k] = dir[k] * force;
     }
-    T d2 = T(0);
-#pragma unroll
-    for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
-    T dist = dsqrt<T>(d2);
-    const bool beyond = cut < 0 ? (dist > cutoff) : (cut == 0);
-    if (beyond || dist == T(0)) {
-#pragma unroll
-        for (int k = 0; k < D; k++) f[k] = T(0);
-        return;
-    }
-    T e = dexp<T>((-stiffness) * (dist - two_radius));
-    T force = ((((T(-2)) * strength) * stiffness) * e) * (T(1) - e);
-#pragma unroll
-    for (int k = 0; k < D; k++) f[k] = (z[k] / dist) * force;
 }
 
 // Float Mie pair path: 1/r from v_rsq_f32 and one Newton step serves sigma / r and
@@ -137,7 +211,7 @@ __device__ __forceinline__ void morse(const T* z, T two_radius, T cutoff, T stre
 // 8.0e-6 with sqrtf and divisions (a drift set by the few agents near unstable
 // equilibria, which any change of rounding tips differently; the force error on
 // the end state is 1.1e-6 RMS either way).
-template <int D>
+template <int D, bool POW>
 __device__ __forceinline__ bool mie_fast(const float* z, const PotParams<float>& P, int cut, float* f) {
     FastDist q;
     q.d2 = 0.0f;
@@ -156,8 +230,9 @@ __device__ __forceinline__ bool mie_fast(const float* z, const PotParams<float>&
         return q.d2 == 0.0f;
     }
     const float sr = P.mie_sigma * q.inv;
-    const float part =
-        P.mie_en_s * powe<float>(sr, P.en + 1.0f, P.ien1) - P.mie_em_s * powe<float>(sr, P.em + 1.0f, P.iem1);
+    float pn, pm;
+    mie_powers<POW>(sr, P, pn, pm);
+    const float part = P.mie_en_s * pn - P.mie_em_s * pm;
     const float force = fminf(P.mie_constant * P.strength * part, P.bound);
     const float fi = force * q.inv;
 #pragma unroll
@@ -168,31 +243,37 @@ __device__ __forceinline__ bool mie_fast(const float* z, const PotParams<float>&
 // MiePotential::calculate_force_between, interaction.rs:345-376.
 // sigma and the Mie constant are pair-independent and precomputed on the host
 // with the reference's expressions.
-template <typename T, int D>
+template <typename T, int D, bool POW>
 __device__ __forceinline__ bool mie(const T* z, const PotParams<T>& P, int cut, T* f) {
-    if constexpr (std::is_same<T, float>::value) return mie_fast<D>(z, P, cut, f);
-    T d2 = T(0);
+    if constexpr (std::is_same<T, float>::value) {
+        return mie_fast<D, POW>(z, P, cut, f);
+    } else {
+        double d2 = 0.0;
 #pragma unroll
-    for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
-    T r = dsqrt<T>(d2);
-    if (r == T(0)) {
+        for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
+        const RootInv q = root_inv(d2);
+        if (q.r == 0.0) {
 #pragma unroll
-        for (int k = 0; k < D; k++) f[k] = T(0);
-        return true;
-    }
-    const bool beyond = cut < 0 ? (r > P.cutoff) : (cut == 0);
-    if (beyond) {
+            for (int k = 0; k < D; k++) f[k] = 0.0;
+            return true;
+        }
+        const bool beyond = cut < 0 ? (q.r > P.cutoff) : (cut == 0);
+        if (beyond) {
 #pragma unroll
-        for (int k = 0; k < D; k++) f[k] = T(0);
+            for (int k = 0; k < D; k++) f[k] = 0.0;
+            return false;
+        }
+        const double sr = param_over(P.mie_sigma, q);
+        double pn, pm;
+        mie_powers<POW>(sr, P, pn, pm);
+        const double part = P.mie_en_s * pn - P.mie_em_s * pm;
+        const double force = fmin(P.mie_constant * P.strength * part, P.bound);
+        double dir[D];
+        direction<D>(z, q, dir);
+#pragma unroll
+        for (int k = 0; k < D; k++) f[k] = dir[k] * force;
         return false;
     }
-    T sr = P.mie_sigma / r;
-    T part = P.en / P.mie_sigma * powe<T>(sr, P.en + T(1), P.ien1) -
-             P.em / P.mie_sigma * powe<T>(sr, P.em + T(1), P.iem1);
-    T force = dmin<T>(P.mie_constant * P.strength * part, P.bound);
-#pragma unroll
-    for (int k = 0; k < D; k++) f[k] = (z[k] / r) * force;
-    return false;
 }
 
 // Float path: 1/r from v_rsq_f32 and one Newton step for sigma / r, 4 epsilon / r,
@@ -220,20 +301,24 @@ template <typename T, int D>
 __device__ __forceinline__ void bound_lj(const T* z, const PotParams<T>& P, int cut, T* f) {
     if constexpr (std::is_same<T, float>::value) {
         bound_lj_fast<D>(z, P, cut, f);
-        return;
+    } else {
+        double d2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
+        const RootInv q = root_inv(d2);
+        const double r = q.r;
+        const double sr = param_over(P.sigma, q);
+        const double er = param_over(4.0 * P.epsilon, q);
+        const double mx = param_over(P.bound, q);
+        const double val = er * (12.0 * ipow<double>(sr, 11) - 6.0 * ipow<double>(sr, 5));
+        const bool inside = cut < 0 ? (P.cutoff >= r) : (cut == 1);
+        const double in = inside ? 1.0 : 0.0;
+        const double m = fmin(mx, val);
+        double dir[D];
+        direction<D>(z, q, dir);
+#pragma unroll
+        for (int k = 0; k < D; k++) f[k] = ((-dir[k]) * in) * m;
     }
-    T d2 = T(0);
-#pragma unroll
-    for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
-    T r = dsqrt<T>(d2);
-    T sr = P.sigma / r;
-    T val = T(4) * P.epsilon / r * (T(12) * ipow<T>(sr, 11) - T(6) * ipow<T>(sr, 5));
-    T mx = P.bound / r;
-    const bool inside = cut < 0 ? (P.cutoff >= r) : (cut == 1);
-    T q = inside ? T(1) : T(0);
-    T m = dmin<T>(mx, val);
-#pragma unroll
-    for (int k = 0; k < D; k++) f[k] = ((-(z[k] / r)) * q) * m;
 }
 
 // CellSpecificInteraction, benchmarks/src/cell_sorting.rs:31-94 (sign +1) and
@@ -290,48 +375,49 @@ template <typename T, int D>
 __device__ __forceinline__ void cell_sorting(const T* z, bool same, const PotParams<T>& P, int cut, T* f) {
     if constexpr (std::is_same<T, float>::value) {
         cell_sorting_fast<D>(z, same, P, cut, f);
-        return;
-    }
-    const T mrd = T(0.3162277660168379);
-    T d2 = T(0);
-#pragma unroll
-    for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
-    T nz = dsqrt<T>(d2);
-    T r;
-    if (!(nz < P.radius * mrd)) {
-        r = nz;
     } else {
-        bool zero = true;
+        const double mrd = 0.3162277660168379;
+        double d2 = 0.0;
 #pragma unroll
-        for (int k = 0; k < D; k++) zero = zero && (z[k] == T(0));
-        if (zero) {
+        for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
+        const RootInv q = root_inv(d2);
+        double r;
+        if (!(q.r < P.radius * mrd)) {
+            r = q.r;
+        } else {
+            bool zero = true;
 #pragma unroll
-            for (int k = 0; k < D; k++) f[k] = T(0);
-            return;
+            for (int k = 0; k < D; k++) zero = zero && (z[k] == 0.0);
+            if (zero) {
+#pragma unroll
+                for (int k = 0; k < D; k++) f[k] = 0.0;
+                return;
+            }
+            r = P.radius * mrd;
         }
-        r = P.radius * mrd;
-    }
-    T sigma = r / P.two_radius;
-    T bound = T(4) + T(1) / sigma;
-    T spatial_cutoff;
-    if (cut < 0) {
-        T sgn_arg = P.rel_range * P.two_radius - r;
-        T signum = (sgn_arg != sgn_arg) ? sgn_arg : copysign(T(1), sgn_arg);
-        spatial_cutoff = (T(1) + signum) * T(0.5);
-    } else {
-        spatial_cutoff = cut ? T(1) : T(0);
-    }
-    T inv = T(1) / sigma;
-    T inv2 = inv * inv;
-    T strength = P.strength * dmax<T>(dmin<T>(inv2 - inv2 * inv2, bound), -bound);
-    T smax = dmax<T>(strength, T(0)), smin = dmin<T>(strength, T(0));
+        const double sigma = over(r, P.two_radius, P.inv_two_radius, q.fast);
+        const double inv = 1.0 / sigma;
+        const double bound = 4.0 + inv;
+        double spatial_cutoff;
+        if (cut < 0) {
+            const double sgn_arg = P.rel_range * P.two_radius - r;
+            const double signum = (sgn_arg != sgn_arg) ? sgn_arg : copysign(1.0, sgn_arg);
+            spatial_cutoff = (1.0 + signum) * 0.5;
+        } else {
+            spatial_cutoff = cut ? 1.0 : 0.0;
+        }
+        const double inv2 = inv * inv;
+        const double strength = P.strength * fmax(fmin(inv2 - inv2 * inv2, bound), -bound);
+        const double smax = fmax(strength, 0.0), smin = fmin(strength, 0.0);
+        double dir[D];
+        direction<D>(z, q, dir);
 #pragma unroll
-    for (int k = 0; k < D; k++) {
-        T dir = z[k] / nz;
-        T att = (dir * smax) * spatial_cutoff;
-        T rep = (dir * smin) * spatial_cutoff;
-        T o = same ? rep + att : rep;
-        f[k] = P.sign < T(0) ? -o : o;
+        for (int k = 0; k < D; k++) {
+            const double att = (dir[k] * smax) * spatial_cutoff;
+            const double rep = (dir[k] * smin) * spatial_cutoff;
+            const double o = same ? rep + att : rep;
+            f[k] = P.sign < 0.0 ? -o : o;
+        }
     }
 }
 
@@ -346,6 +432,7 @@ __device__ __forceinline__ void cell_sorting(const T* z, bool same, const PotPar
 template <typename T, int D>
 __device__ __forceinline__ void sorting_langevin(const T* z, T attraction, const PotParams<T>& P, int cut, T* f) {
     T d2 = T(0), r, inv;
+    RootInv root{};
     if constexpr (std::is_same<T, float>::value) {
         const FastDist q = fast_dist<D>(z);
         d2 = q.d2;
@@ -354,7 +441,8 @@ __device__ __forceinline__ void sorting_langevin(const T* z, T attraction, const
     } else {
 #pragma unroll
         for (int k = 0; k < D; k++) d2 = d2 + z[k] * z[k];
-        r = dsqrt<T>(d2);
+        root = root_inv(d2);
+        r = root.r;
         inv = T(0);
     }
     if (d2 == T(0)) {  // dir = 0
@@ -367,21 +455,28 @@ __device__ __forceinline__ void sorting_langevin(const T* z, T attraction, const
     if (r <= R) {
         s = P.strength * (R - r);
     } else if (cut < 0 ? (r <= P.cutoff) : (cut == 1)) {
-        const T sm1 = r / R - T(1);
-        T e;
-        if constexpr (std::is_same<T, float>::value) e = __expf(-(sm1 * sm1));
-        else e = dexp<T>(T(-1) * (sm1 * sm1));
-        s = ((((-attraction) * (r - R)) * (P.cutoff - r)) / P.cutoff) * e;
+        const T pull = ((-attraction) * (r - R)) * (P.cutoff - r);
+        if constexpr (std::is_same<T, float>::value) {
+            const T sm1 = r / R - T(1);
+            s = (pull / P.cutoff) * __expf(-(sm1 * sm1));
+        } else {
+            const T sm1 = over(r, R, P.inv_two_radius, root.fast) - T(1);
+            s = over(pull, P.cutoff, P.inv_cutoff, root.fast) * exp(T(-1) * (sm1 * sm1));
+        }
     } else {
 #pragma unroll
         for (int k = 0; k < D; k++) f[k] = T(0);
         return;
     }
+    T dir[D];
+    if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
-    for (int k = 0; k < D; k++) {
-        if constexpr (std::is_same<T, float>::value) f[k] = -(s * (z[k] * inv));
-        else f[k] = -(s * (z[k] / r));
+        for (int k = 0; k < D; k++) dir[k] = z[k] * inv;
+    } else {
+        direction<D>(z, root, dir);
     }
+#pragma unroll
+    for (int k = 0; k < D; k++) f[k] = -(s * dir[k]);
 }
 
 // Radius at which the potential is discontinuous (the cutoff test).
@@ -415,8 +510,8 @@ __device__ __forceinline__ bool point_force(const T* z, bool same, T strength, c
     if constexpr (POT == CRM_POTENTIAL_MORSE || POT == CRM_POTENTIAL_MORSE_SPECIES) {
         morse<T, D>(z, P.two_radius, P.cutoff, strength, P.stiffness, cut, f);
         return false;
-    } else if constexpr (POT == CRM_POTENTIAL_MIE) {
-        return mie<T, D>(z, P, cut, f);
+    } else if constexpr (POT == CRM_POTENTIAL_MIE || POT == kPotentialMiePow) {
+        return mie<T, D, POT == kPotentialMiePow>(z, P, cut, f);
     } else if constexpr (POT == CRM_POTENTIAL_BOUND_LENNARD_JONES) {
         bound_lj<T, D>(z, P, cut, f);
         return false;
@@ -431,12 +526,6 @@ __device__ __forceinline__ bool point_force(const T* z, bool same, T strength, c
         cell_sorting<T, D>(z, same, P, cut, f);
         return false;
     }
-}
-
-// Strength of the (own, ext) species pair from a row of the matrix held in registers.
-template <typename T>
-__device__ __forceinline__ T pick4(const T* row, int k) {
-    return k == 0 ? row[0] : (k == 1 ? row[1] : (k == 2 ? row[2] : row[3]));
 }
 
 // nearest_point_from_point_to_line, interaction.rs:497-509 (t and the point x).

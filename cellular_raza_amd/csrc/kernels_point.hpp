@@ -524,7 +524,10 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
         calc_err |= point_force<POT, T, D>(z, same_sp, srow.pick(sp_j), PP, cut, f);
         T wgt = T(0.5);
         if (full) {
-            if (symmetric) {
+            // (only interactions of species pairs can differ by the order of the pair)
+            constexpr bool by_species =
+                POT == CRM_POTENTIAL_MORSE_SPECIES || POT == CRM_POTENTIAL_CELL_SORTING_LANGEVIN;
+            if (!by_species || symmetric) {
                 wgt = T(1);
             } else {
                 T zj[D], g[D];
