@@ -174,12 +174,13 @@ enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 // 4.5 GB/s (page faults), two at 8, four at 12.5, eight at 19-20 GB/s (48 MB and
 // 192 MB; the link carries 55 GB/s).  Read-backs above kPinLarge get kPinChunkLarge
 // chunks, allocated on the first one (48 MB: 2.7 ms in either size, 192 MB: 9.9 ms
-// against 10.9 with half of it); an allocation takes 0.1 ms up to 2 MB, 0.3 ms at 8.
+// against 10.9 with half of it; 8 MB: 0.59 against 0.76 ms in small chunks); an
+// allocation takes 0.1 ms up to 2 MB, 0.3 ms at 8.
 constexpr size_t kPinControl = 4096;
 constexpr uint32_t kPinWorkers = 8;
 constexpr size_t kPinChunkSmall = 256 * 1024;
 constexpr size_t kPinChunkLarge = 1024 * 1024;
-constexpr size_t kPinLarge = 8 * 1024 * 1024;
+constexpr size_t kPinLarge = 4 * 1024 * 1024;
 // Largest read-back that the kernel writes to pinned memory itself: get_state takes
 // 36 us at 259 KB, and 94 us at 269 KB through two host threads (256 KB and more to a
 // thread is where a second one pays for its start).
@@ -230,6 +231,8 @@ struct crm_ctx {
     uint32_t n_force_tiles = 0;
     size_t tiles_cap = 0;
     uint32_t policy = 0;                  // tiling policy (index into kTilePolicies)
+    bool policy_tuned = false;            // chosen by crm_autotune (else default_policy)
+    uint32_t n_cu = 0;
     uint32_t lanes_log2 = 0;              // lanes per own agent in the force kernel (policy's)
     std::vector<uint32_t> tile_rows, tile_cols, tile_count;  // per instance
     Control* d_ctrl = nullptr;
@@ -859,7 +862,7 @@ crm_status reset_control(crm_ctx* ctx, uint64_t step) {
 // the smallest region.
 // Tiling policies the autotuner chooses from: the fraction of the workgroup's
 // lanes the expected own agents may fill, and the density margin on the staged
-// region.  Policy 0 is the default.
+// region.  Contexts that are not tuned take default_policy.
 // own_frac: the tile's expected own agents per lane of the workgroup (above 1, a
 // lane walks several own agents one after another, which fills the lanes of
 // tiles cut from small grids)
@@ -873,8 +876,12 @@ constexpr TilePolicy kTilePolicies[] = {{0.94, 1.2, 0}, {0.94, 1.1, 0}, {0.94, 1
                                         {1.50, 1.2, 0}, {1.90, 1.2, 0}, {0.94, 1.2, 3}, {0.70, 1.2, 3}};
 constexpr uint32_t kNumTilePolicies = sizeof(kTilePolicies) / sizeof(kTilePolicies[0]);
 
-void build_tiles(const InstParams& P, uint32_t dim, uint32_t inst, uint64_t n_agents, uint32_t cap,
-                 const TilePolicy& pol, std::vector<ForceTile>& out, uint32_t& rows, uint32_t& cols_out) {
+struct TileShape {
+    uint32_t rows, cols;
+    uint64_t tiles;
+};
+
+TileShape tile_shape(const InstParams& P, uint32_t dim, uint64_t n_agents, uint32_t cap, const TilePolicy& pol) {
     const uint32_t n0 = P.n[0], n1 = P.n[1], n2 = P.n[2];
     const double rho = (double)n_agents / ((double)n0 * n1 * n2);
     const uint32_t np = dim == 3 ? 3u : 1u;  // staged planes
@@ -901,12 +908,38 @@ void build_tiles(const InstParams& P, uint32_t dim, uint32_t inst, uint64_t n_ag
             }
         }
     }
-    for (uint32_t a = 0; a < n0; a++)
-        for (uint32_t b = 0; b < n1; b += bR)
-            for (uint32_t c = 0; c < n2; c += bW)
-                out.push_back(ForceTile{inst, a, b, std::min(b + bR, n1), c, std::min(c + bW, n2)});
-    rows = bR;
-    cols_out = bW;
+    return TileShape{bR, bW, (uint64_t)n0 * ((n1 + bR - 1) / bR) * ((n2 + bW - 1) / bW)};
+}
+
+uint32_t tile_cap(const crm_ctx* ctx) {  // staged records that fit a tile's LDS
+    const bool mixed = ctx->cfg.precision == CRM_PRECISION_MIXED;
+    return ctx->D == 2 ? (mixed ? LdsRecords<2, true>::kCap : LdsRecords<2, false>::kCap)
+                       : (mixed ? LdsRecords<3, true>::kCap : LdsRecords<3, false>::kCap);
+}
+
+// Tiling policy of a context that has not been tuned: the most lanes per agent whose
+// tiles all run at once -- 4 (FP64) or 5 (mixed) workgroups per CU, 3 with 8 lanes,
+// where every tile's set-up serves few agents.  A system whose one-lane tiles leave
+// most of the chip idle runs as long as its longest lane, which several lanes per
+// agent shorten: force kernel with one lane / by this rule, event-timed: 1000 2-D
+// agents 21.8 / 14.6 us, 1600 crowded 3-D agents (FP64) 66 / 29, 20,480 benchmark
+// cells 36.4 / 25.1, 30,000 sorting agents 21.9 / 19.3 (mixed 20.1 / 16.6), 60,000
+// 31.7 / 22.9.  Beyond the line the set-up costs more than it hides: 100,000 FP64
+// agents take 27.6 us with one lane and 32.4 in 1188 two-lane tiles, 30,000 mixed
+// ones 16.6 with four lanes and 21.3 in 1450 eight-lane tiles.
+uint32_t default_policy(const crm_ctx* ctx) {
+    if (is_rod(ctx) || (ctx->cfg.flags & CRM_FLAG_NO_LDS)) return 0;
+    const uint32_t cap = tile_cap(ctx);
+    const uint64_t resident = (uint64_t)ctx->n_cu * (ctx->cfg.precision == CRM_PRECISION_MIXED ? 5 : 4);
+    for (uint32_t pol : {15u, 11u, 9u}) {
+        const TilePolicy& T = kTilePolicies[pol];
+        const uint64_t most = T.lanes_log2 == 3 ? (uint64_t)ctx->n_cu * 3 : resident;
+        uint64_t tiles = 0;
+        for (uint32_t i = 0; i < ctx->n_inst && tiles <= most; i++)
+            tiles += tile_shape(ctx->hparams[i], ctx->D, ctx->counts[i], cap, T).tiles;
+        if (tiles <= most) return pol;
+    }
+    return 0;
 }
 
 template <typename T>
@@ -917,16 +950,22 @@ crm_status dalloc(crm_ctx* ctx, T*& p, size_t n) {
 
 // Force tiles of every instance under tiling policy `pol`.
 void make_tiles(crm_ctx* ctx, uint32_t pol, std::vector<ForceTile>& tiles) {
-    const uint32_t cap = ctx->cfg.precision == CRM_PRECISION_MIXED ? kLdsRecordsMixed : kLdsRecordsFP64;
+    const uint32_t cap = tile_cap(ctx);
     tiles.clear();
     ctx->tile_rows.assign(ctx->n_inst, 0);
     ctx->tile_cols.assign(ctx->n_inst, 0);
     ctx->tile_count.assign(ctx->n_inst, 0);
     for (uint32_t i = 0; i < ctx->n_inst; i++) {
-        const size_t before = tiles.size();
-        build_tiles(ctx->hparams[i], ctx->D, i, ctx->counts[i], cap, kTilePolicies[pol], tiles, ctx->tile_rows[i],
-                    ctx->tile_cols[i]);
-        ctx->tile_count[i] = (uint32_t)(tiles.size() - before);
+        const InstParams& P = ctx->hparams[i];
+        const TileShape T = tile_shape(P, ctx->D, ctx->counts[i], cap, kTilePolicies[pol]);
+        const uint32_t n0 = P.n[0], n1 = P.n[1], n2 = P.n[2];
+        for (uint32_t a = 0; a < n0; a++)
+            for (uint32_t b = 0; b < n1; b += T.rows)
+                for (uint32_t c = 0; c < n2; c += T.cols)
+                    tiles.push_back(ForceTile{i, a, b, std::min(b + T.rows, n1), c, std::min(c + T.cols, n2)});
+        ctx->tile_rows[i] = T.rows;
+        ctx->tile_cols[i] = T.cols;
+        ctx->tile_count[i] = (uint32_t)T.tiles;
     }
     ctx->lanes_log2 = kTilePolicies[pol].lanes_log2;
 }
@@ -1921,6 +1960,10 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
     ctx->device = cfg->device;
     hipError_t e = hipSetDevice(cfg->device);
     if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipSetDevice: ") + hipGetErrorString(e));
+    int n_cu = 0;
+    e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, cfg->device);
+    if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipDeviceGetAttribute: ") + hipGetErrorString(e));
+    ctx->n_cu = (uint32_t)n_cu;
     e = scratch_address(cfg->device, ctx->d_noalloc);
     if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
     ctx->inst_host.assign(n_instances, 0);
@@ -1991,6 +2034,7 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
     }
     ctx->n_work = (uint32_t)work.size();
     std::vector<ForceTile> tiles;
+    if (!ctx->policy_tuned) ctx->policy = default_policy(ctx);
     make_tiles(ctx, ctx->policy, tiles);
     CRM_HIP(hipMemcpy(ctx->d_ip, ctx->hparams.data(), sizeof(InstParams) * ctx->n_inst, hipMemcpyHostToDevice));
 
@@ -2366,6 +2410,7 @@ crm_status apply_policy(crm_ctx* ctx, uint32_t pol) {
     make_tiles(ctx, pol, tiles);
     CRM_TRY(upload_tiles(ctx, tiles));
     ctx->policy = pol;
+    ctx->policy_tuned = true;
     for (auto& g : ctx->graph)  // captured with the old tile table
         if (g) {
             (void)hipGraphExecDestroy(g);

@@ -208,11 +208,49 @@ struct Walk3 {
     }
 };
 
+// Staged records in LDS, addressed by the byte offset kBytes * index: int4 (mixed), or
+// one array of doubles per axis (FP64; the species are bytes beside them).  The
+// capacities keep the occupancy the registers allow: 5 workgroups of at most 32000 bytes
+// per CU (mixed; LDS is given out in 1280-byte granules, and 32512 bytes cost the// fifth), 4 of at most 40960 (FP64).  The FP64 records were double4 (896 of
+// them) and the mixed ones 1024: LDS bounded the tiles, whose own agents filled 64 %
+// of the lanes on the 4M-agent lattice (now 84 %).
+template <int D, bool MIXED>
+struct LdsRecords;
+template <int D>
+struct LdsRecords<D, true> {
+    static constexpr int kCap = 1232;
+    static constexpr uint32_t kBytes = sizeof(int4);
+    static constexpr uint32_t kTotal = kCap * kBytes;
+    static __device__ __forceinline__ int4 at(const char* lds, uint32_t off) {
+        return *reinterpret_cast<const int4*>(lds + off);
+    }
+    static __device__ __forceinline__ void put(char* lds, uint32_t j, const int4 r) {
+        *reinterpret_cast<int4*>(lds + j * kBytes) = r;
+    }
+};
+template <int D>
+struct LdsRecords<D, false> {
+    static constexpr int kCap = D == 3 ? 1152 : 1600;  // multiples of 64 (ds_read2st64 pairs two axes)
+    static constexpr uint32_t kBytes = sizeof(double);
+    static constexpr uint32_t kTotal = kCap * kBytes * D;
+    static __device__ __forceinline__ double4 at(const char* lds, uint32_t off) {
+        const double* x = reinterpret_cast<const double*>(lds + off);
+        return make_double4(x[0], x[kCap], D == 3 ? x[(D - 1) * kCap] : 0.0, 0.0);
+    }
+    static __device__ __forceinline__ void put(char* lds, uint32_t j, const double4 r) {
+        double* x = reinterpret_cast<double*>(lds) + j;
+        x[0] = r.x;
+        x[kCap] = r.y;
+        if constexpr (D == 3) x[2 * kCap] = r.z;
+    }
+};
+
 template <int D, bool MIXED>
 struct LdsSource {
     using Rec = typename RecOf<MIXED>::type;
     using W = Walk3;
-    const Rec* lds;       // staged records, converted
+    const char* lds;      // staged records, converted (LdsRecords)
+    const uint8_t* lsp;   // FP64: species of each staged record
     const uint16_t* vst;  // LDS index of the first agent of staged voxel v; vst[n_vox] = total
     Region G;
     uint32_t np, n_vox;
@@ -224,7 +262,12 @@ struct LdsSource {
     __device__ __forceinline__ uint32_t vox(uint32_t rb, uint32_t c, uint32_t pa) const {
         return (rb * G.NC + (c - G.cl)) * np + pa;
     }
-    __device__ __forceinline__ Rec record(uint32_t j, const W&) const { return lds[j]; }
+    using Recs = LdsRecords<D, MIXED>;
+    __device__ __forceinline__ Rec record(uint32_t j, const W&) const { return Recs::at(lds, j * Recs::kBytes); }
+    __device__ __forceinline__ int species(uint32_t j, const Rec& r) const {
+        if constexpr (MIXED) return (int)((uint32_t)r.w & kSpeciesMask);
+        else return (int)lsp[j];
+    }
     // global slot of LDS index j (only on the rare FP64 re-evaluation path)
     __device__ __forceinline__ uint32_t slot(uint32_t j, const W&) const {
         uint32_t lo = 0, hi = n_vox;  // largest v with vst[v] <= j
@@ -281,6 +324,10 @@ struct GlobalSource {
         else
             return rec[j];
     }
+    __device__ __forceinline__ int species(uint32_t, const Rec& r) const {
+        if constexpr (MIXED) return (int)((uint32_t)r.w & kSpeciesMask);
+        else return (int)r.w;
+    }
     __device__ __forceinline__ uint32_t slot(uint32_t j, const W&) const { return j; }
     __device__ __forceinline__ uint32_t sub_of(uint32_t, const W& w, const InstParams& P) const {
         return subdomain_of(P, w.gvox() - w.voff);
@@ -314,8 +361,10 @@ struct Row4 {
 // instead of max-over-lanes of the candidate count.
 //
 // Lanes per agent (LDS source): 2^lg consecutive lanes of a wave share one agent;
-// lane `sub` of the group walks the sub-th of 2^lg equal parts of the stream, and
-// the group adds its partial sums with wavefront shuffles (a butterfly, so every
+// lane `sub` of the group walks every 2^lg-th candidate of the stream from the sub-th
+// (a cluster of close agents is spread over the lanes; with one contiguous part per
+// lane 2400 crowded 3-D agents that had drawn together took 164 us with 8 lanes and
+// 92 with one), and the group adds its partial sums with wavefront shuffles (a butterfly, so every
 // lane of the group holds the same total) before lane 0 writes the force.
 template <int D, int POT, bool MIXED, bool SENSE, typename Src>
 __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, const InstParams& P, uint64_t s,
@@ -331,14 +380,9 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
     const float rc2 = (float)(rc * rc);
     const float band = 2e-6f * rc2;
 
-    int sp_i;
+    const int sp_i = src.species(self, me);
     bool flag_i = false;
-    if constexpr (MIXED) {
-        sp_i = (int)((uint32_t)me.w & kSpeciesMask);
-        flag_i = me.w < 0;
-    } else {
-        sp_i = (int)me.w;
-    }
+    if constexpr (MIXED) flag_i = me.w < 0;
     // candidate test thresholds: mixed marks d2 <= rc2 + band (the band pairs are
     // re-decided in FP64) and every pair with a flagged agent; FP64 marks
     // d2 <= rc^2 (1 + 1e-12), beyond which the rounded sqrt(d2) exceeds rc.
@@ -500,10 +544,9 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
             }
         }
         const bool full = physical || (j >= ov.b && j < ov.e) || (subs && src.sub_of(j, w, P) != my_sub);
-        int sp_j;
+        const int sp_j = src.species(j, rj);
         int cut = -1;
         if constexpr (MIXED) {
-            sp_j = (int)((uint32_t)rj.w & kSpeciesMask);
             const bool refine = flag_i || rj.w < 0 || d2 < close2 || fabsf(d2 - rc2) <= band;
             if (refine) {
                 const uint32_t gj = src.slot(j, w);
@@ -516,8 +559,6 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
                 }
                 cut = cut_decision<POT>(P.pd, sqrt(dd));
             }
-        } else {
-            sp_j = (int)rj.w;
         }
         T f[D];
         const bool same_sp = sp_i == sp_j;
@@ -560,22 +601,21 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
         const uint32_t B1 = cur.je - cur.j, B2 = B1 + (cur.e1 - cur.j1);
         const uint32_t L = active ? B2 + (cur.e2 - cur.j2) : 0u;
         const uint32_t o1 = cur.j1 - cur.je, o2 = cur.j2 - cur.e1;  // modular offsets
-        // this lane's part [pb, pe) of the stream, walked by the offset r = p - pb
+        // this lane's share of the stream, the positions p = sub + (r << lg), walked by r
         // (the same for every lane of a wave, so the loop counters stay scalar)
-        const uint32_t part = (L + (1u << lg) - 1u) >> lg;
-        const uint32_t pb = min(L, sub * part), Lr = min(L, pb + part) - pb;
-        const uint32_t j0 = cur.j + pb + (pb >= B1 ? o1 : 0u) + (pb >= B2 ? o2 : 0u);
-        // range boundaries ahead of the part's start, and their offsets
-        const uint32_t R1 = B1 > pb ? B1 - pb : 0u, R2 = B2 > pb ? B2 - pb : 0u;
-        const uint32_t off1 = pb < B1 ? o1 : 0u, off2 = pb < B2 ? o2 : 0u;
-        const uint32_t r_self = B1 + (self - cur.j1) - pb;  // wraps above Lr when before the part
+        const uint32_t last = (1u << lg) - 1u;
+        auto upto = [&](uint32_t e) -> uint32_t { return e > sub ? (e - sub + last) >> lg : 0u; };
+        const uint32_t Lr = upto(L);
+        const uint32_t R1 = upto(B1), R2 = upto(B2);  // first r of the later ranges
+        const uint32_t p_self = B1 + (self - cur.j1);
+        const uint32_t r_self = (p_self & last) == sub ? p_self >> lg : 0xffffffffu;
         // LDS byte offset of stream offset r (the range offsets scaled once, not per
         // candidate), its record and its LDS index
-        constexpr uint32_t RB = (uint32_t)sizeof(Rec);
-        const uint32_t jb0 = j0 * RB, off1b = off1 * RB, off2b = off2 * RB;
-        const char* lds_b = reinterpret_cast<const char*>(src.lds);
-        auto atb = [&](uint32_t r) -> uint32_t { return jb0 + r * RB + (r >= R1 ? off1b : 0u) + (r >= R2 ? off2b : 0u); };
-        auto rec_at = [&](uint32_t r) -> Rec { return *reinterpret_cast<const Rec*>(lds_b + atb(r)); };
+        using Recs = typename Src::Recs;
+        constexpr uint32_t RB = Recs::kBytes;
+        const uint32_t jb0 = (cur.j + sub) * RB, off1b = o1 * RB, off2b = o2 * RB, RS = RB << lg;
+        auto atb = [&](uint32_t r) -> uint32_t { return jb0 + r * RS + (r >= R1 ? off1b : 0u) + (r >= R2 ? off2b : 0u); };
+        auto rec_at = [&](uint32_t r) -> Rec { return Recs::at(src.lds, atb(r)); };
         auto at = [&](uint32_t r) -> uint32_t { return atb(r) / RB; };
         // unit grids (equal fixed-point steps on every axis) need no axis scaling in
         // pass 1 (r1 = r2 = 1 exactly, so the marks are the same)
@@ -699,8 +739,6 @@ __device__ __forceinline__ void agent_force(const Arrays& A, const StateBuf& S, 
 
 // A force tile: plane a0, rows [b0, b1), columns [c0, c1) of one instance.
 constexpr int kTileRowsMax = 29;
-constexpr int kLdsRecordsMixed = 1024;  // 16 KiB of int4
-constexpr int kLdsRecordsFP64 = 896;    // 28 KiB of double4
 constexpr int kLdsVoxelStarts = 768;    // 1.5 KiB of voxel-start indices (staged voxels + 1)
 constexpr int kOwnVoxMax = 256;         // own voxels per tile
 constexpr int kSortBins = 64;           // candidate-count classes for the lane order
@@ -768,12 +806,14 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                                                                      uint32_t lanes_log2) {
     const uint32_t lg = MULTI ? lanes_log2 : 0u;
     using Rec = typename RecOf<MIXED>::type;
-    constexpr int CAP = MIXED ? kLdsRecordsMixed : kLdsRecordsFP64;
+    using Recs = LdsRecords<D, MIXED>;
+    constexpr int CAP = Recs::kCap;
     constexpr uint32_t NP = D == 3 ? 3u : 1u;         // staged planes
     const ForceTile T = tiles[xcd_block(blockIdx.x, gridDim.x)];  // loaded beside the control block
     if (halted(A.ctrl, A.ctrl->step)) return;
     constexpr uint32_t PA_OWN = D == 3 ? 1u : 0u;     // the tile's own plane among them
-    __shared__ Rec lds[CAP];
+    __shared__ __align__(16) char lds[Recs::kTotal];
+    __shared__ uint8_t lsp[MIXED ? 1 : CAP];         // FP64: species of each staged record
     __shared__ uint16_t vst[kLdsVoxelStarts];        // LDS index of each staged voxel's first agent
     __shared__ uint16_t own_pre[kOwnVoxMax + 1];     // own agents before own voxel u
     __shared__ uint32_t own_gs[kOwnVoxMax];          // global slot of own voxel u's first agent
@@ -896,8 +936,12 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                     const uint32_t pa = (uint32_t)pa_q[q], rb = (uint32_t)rb_q[q], c = c_q[q];
                     for (uint32_t k = 0; k < cnt[q]; k++) {
                         const Rec r = k < kPreRecs ? pre[q][k] : rec[gs[q] + k];
-                        if constexpr (MIXED) lds[run + k] = to_region<D>(r, (int)pa, (int)rb, G);
-                        else lds[run + k] = r;
+                        if constexpr (MIXED) {
+                            Recs::put(lds, run + k, to_region<D>(r, (int)pa, (int)rb, G));
+                        } else {
+                            Recs::put(lds, run + k, r);
+                            lsp[run + k] = (uint8_t)(int)r.w;
+                        }
                     }
                     if (P.sub_on && cnt[q]) {
                         const int a = (int)T.a0 + (int)pa - (int)PA_OWN, b = (int)T.b0 - 1 + (int)rb;
@@ -927,7 +971,7 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
             }
             __syncthreads();
             const uint32_t n_own = own_pre[n_ownv];
-            LdsSource<D, MIXED> src{lds, vst, G, NP, n_vox, A.start, voff, n1, n2, lsub};
+            LdsSource<D, MIXED> src{lds, lsp, vst, G, NP, n_vox, A.start, voff, n1, n2, lsub};
             const float inv_w = 1.0f / (float)W;
             // own agent t: own voxel u (largest u with own_pre[u] <= t), LDS index,
             // global slot, and the three ranges of its stream
@@ -1005,7 +1049,8 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                     w.j2 = e.r[4];
                     w.e2 = e.r[5];
                     w.left = 2;
-                    agent_force<D, POT, MIXED, SENSE>(A, S, P, e.slot, e.self, lds[e.self], Span{e.ovb, e.ove}, w,
+                    agent_force<D, POT, MIXED, SENSE>(A, S, P, e.slot, e.self, src.record(e.self, w),
+                                                      Span{e.ovb, e.ove}, w,
                                                       physical, symmetric, src, unit, MULTI ? threadIdx.x & gmask : 0u,
                                                       lg);
                 }
@@ -1017,7 +1062,7 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                 Span ov;
                 Walk3 w;
                 const uint32_t s = own_agent(t >> lg, self, ov, w);
-                agent_force<D, POT, MIXED, SENSE>(A, S, P, s, self, lds[self], ov, w, physical, symmetric, src, unit,
+                agent_force<D, POT, MIXED, SENSE>(A, S, P, s, self, src.record(self, w), ov, w, physical, symmetric, src, unit,
                                                   MULTI ? t & gmask : 0u, lg);
             }
             rank_tile(true);

@@ -1,6 +1,6 @@
 """Read-backs in agent order on every transfer path: rows written to pinned memory by
 the gathering kernel (up to 256 KiB), chunks of 256 KiB through host threads, and
-chunks of 1 MiB (above 8 MiB), at the sizes next to each limit.  The state read right
+chunks of 1 MiB (above 4 MiB), at the sizes next to each limit.  The state read right
 after set_agents is the caller's own, bit for bit, although the slots are in voxel
 order; the forces of a spring without pair interactions are -k (x - c) in closed form
 (one product, so exact; the mixed path rounds them once to float)."""
@@ -13,8 +13,8 @@ from cellular_raza_amd import (CartesianCuboid, DomainSpring, InstanceSpec, Mech
 pytestmark = pytest.mark.gpu
 
 # agents of a 3-D system whose positions and velocities (48 bytes) end next to 256 KiB,
-# to eight chunks of 256 KiB, and to 8 MiB
-SIZES = [1, 5461, 5462, 43690, 43691, 174762, 174763, 400001]
+# to eight chunks of 256 KiB, to 4 MiB and to 8 MiB
+SIZES = [1, 5461, 5462, 43690, 43691, 87381, 87382, 174762, 174763, 400001]
 
 
 @pytest.mark.parametrize("n", SIZES)
