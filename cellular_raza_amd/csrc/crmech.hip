@@ -239,7 +239,7 @@ struct crm_ctx {
     uint32_t* d_start = nullptr;
     uint32_t* d_count = nullptr;
     uint32_t* d_start_local = nullptr;  // [Vt] voxel offsets inside their scan tile
-    uint32_t* d_bsum = nullptr;         // [n_tiles] scan tile sums, then offsets
+    uint32_t* d_bsum = nullptr;         // [n_tiles + 1] scan tile sums, then (more than kScatterTiles) offsets, total
     uint32_t n_tiles = 0;
     uint32_t* d_key = nullptr;
     uint32_t* d_rank = nullptr;
@@ -537,7 +537,7 @@ crm_status launch_force_d(crm_ctx* ctx, StateBuf S, uint32_t rank) {
 }
 
 template <int D, bool MIXED>
-crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S) {
+crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S, uint32_t rank) {
     Arrays A = arrays(ctx);
     const RodArgs R = rod_args(ctx);
     const uint32_t phys = ctx->cfg.weighting == CRM_WEIGHT_PHYSICAL;
@@ -545,40 +545,34 @@ crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S) {
     const dim3 g(ctx->n_work), b(kBlock);
     switch (ctx->pot_kind) {
         case CRM_POTENTIAL_MORSE:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
-                               no_lds);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             return CRM_OK;
         case CRM_POTENTIAL_MORSE_SPECIES:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE_SPECIES, MIXED>), g, b, 0, ctx->stream, A, S, R,
-                               phys, no_lds);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE_SPECIES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             return CRM_OK;
         case CRM_POTENTIAL_MIE:
             if (ctx->mie_pow)
-                hipLaunchKernelGGL((k_force_rod<D, kPotentialMiePow, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
-                                   no_lds);
+                hipLaunchKernelGGL((k_force_rod<D, kPotentialMiePow, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             else
-                hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
-                                   no_lds);
+                hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             return CRM_OK;
         case CRM_POTENTIAL_BOUND_LENNARD_JONES:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_BOUND_LENNARD_JONES, MIXED>), g, b, 0, ctx->stream, A, S,
-                               R, phys, no_lds);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_BOUND_LENNARD_JONES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             return CRM_OK;
         case CRM_POTENTIAL_NONE:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_NONE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys,
-                               no_lds);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_NONE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
             return CRM_OK;
     }
     return CRM_INVALID_ARGUMENT;
 }
 
 template <int D>
-crm_status launch_force_rod_d(crm_ctx* ctx, StateBuf S) {
-    return ctx->cfg.precision == CRM_PRECISION_MIXED ? launch_force_rod_dm<D, true>(ctx, S)
-                                                     : launch_force_rod_dm<D, false>(ctx, S);
+crm_status launch_force_rod_d(crm_ctx* ctx, StateBuf S, uint32_t rank) {
+    return ctx->cfg.precision == CRM_PRECISION_MIXED ? launch_force_rod_dm<D, true>(ctx, S, rank)
+                                                     : launch_force_rod_dm<D, false>(ctx, S, rank);
 }
 
-// rank: point agents binned ahead -- the force kernel also ranks the step's
+// rank: agents binned ahead -- the force kernel also ranks the step's
 // re-binning (only inside a step: a force evaluation on its own must leave the
 // histogram alone).
 crm_status launch_force(crm_ctx* ctx, bool rank = false) {
@@ -587,7 +581,7 @@ crm_status launch_force(crm_ctx* ctx, bool rank = false) {
     ctx->sense_parity = ctx->cur;
     crm_status st;
     const uint32_t r = rank ? 1u : 0u;
-    if (is_rod(ctx)) st = ctx->D == 2 ? launch_force_rod_d<2>(ctx, S) : launch_force_rod_d<3>(ctx, S);
+    if (is_rod(ctx)) st = ctx->D == 2 ? launch_force_rod_d<2>(ctx, S, r) : launch_force_rod_d<3>(ctx, S, r);
     else st = ctx->D == 2 ? launch_force_d<2>(ctx, S, r) : launch_force_d<3>(ctx, S, r);
     if (st) return st;
     return t_end(ctx, CRM_KERNEL_FORCE);
@@ -707,20 +701,23 @@ crm_status launch_sort(crm_ctx* ctx, bool advance, const StepArgs* sa) {
         hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kBlock), 0, ctx->stream, A, (uint32_t)(advance ? 1 : 0));
         CRM_TRY(t_end(ctx, CRM_KERNEL_SCAN));
     } else {
+        const bool scan = ctx->n_tiles <= kScatterTiles;  // the scatter scans the tile sums itself
+        const uint32_t adv = advance ? 1u : 0u;
         CRM_TRY(t_begin(ctx));
         hipLaunchKernelGGL(k_scan_local, dim3(ctx->n_tiles), dim3(kBlock), 0, ctx->stream, ctx->d_count,
                            ctx->d_count + stay_offset(ctx), ctx->d_start_local, ctx->d_bsum, Vt, ctx->d_ctrl);
-        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->d_bsum, ctx->n_tiles,
-                           ctx->d_start, Vt, ctx->d_ctrl, (uint32_t)(advance ? 1 : 0));
+        if (!scan)
+            hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->d_bsum, ctx->n_tiles,
+                               ctx->d_ctrl);
         CRM_TRY(t_end(ctx, CRM_KERNEL_SCAN));
         CRM_TRY(t_begin(ctx));
         const uint64_t n_scatter = std::max<uint64_t>(ctx->N, Vt);
-        hipLaunchKernelGGL(k_scatter, dim3((uint32_t)((n_scatter + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                           ctx->stream, A);
+        const dim3 g((uint32_t)((n_scatter + kBlock - 1) / kBlock));
+        if (scan) hipLaunchKernelGGL(k_scatter<true>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles, adv);
+        else hipLaunchKernelGGL(k_scatter<false>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles, adv);
         CRM_TRY(t_end(ctx, CRM_KERNEL_SCATTER));
     }
-    // the point gather of a step orders each voxel's arrivals itself
-    if (is_rod(ctx) || !advance) {
+    if (!advance) {  // the gather of a step orders each voxel's arrivals itself
         CRM_TRY(t_begin(ctx));
         hipLaunchKernelGGL(k_fixup, dim3((Vt + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream, A);
         CRM_TRY(t_end(ctx, CRM_KERNEL_FIXUP));
@@ -783,16 +780,9 @@ bool keys_ahead(const crm_ctx* ctx) {
 
 crm_status launch_step(crm_ctx* ctx, const double* noise_step) {
     const StepArgs sa = step_args(ctx, noise_step);
-    const bool fused_rank = keys_ahead(ctx) && !is_rod(ctx);  // the force tiles rank their voxels
-    CRM_TRY(launch_force(ctx, fused_rank));
-    if (!keys_ahead(ctx)) {
-        CRM_TRY(launch_key(ctx, sa));
-    } else if (!fused_rank) {
-        CRM_TRY(t_begin(ctx));
-        hipLaunchKernelGGL(k_rank_ahead, dim3((uint32_t)((ctx->Vt + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                           ctx->stream, arrays(ctx));
-        CRM_TRY(t_end(ctx, CRM_KERNEL_INTEGRATE));
-    }
+    const bool ahead = keys_ahead(ctx);  // the force kernel ranks the voxels
+    CRM_TRY(launch_force(ctx, ahead));
+    if (!ahead) CRM_TRY(launch_key(ctx, sa));
     CRM_TRY(launch_sort(ctx, true, &sa));
     return CRM_OK;
 }
@@ -2049,7 +2039,7 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
     CRM_TRY(dalloc(ctx, ctx->d_start, Vt + 1));
     CRM_TRY(dalloc(ctx, ctx->d_count, stay_offset(ctx) + Vt));  // arrivals, then stayers
     CRM_TRY(dalloc(ctx, ctx->d_start_local, Vt));
-    CRM_TRY(dalloc(ctx, ctx->d_bsum, ctx->n_tiles));
+    CRM_TRY(dalloc(ctx, ctx->d_bsum, ctx->n_tiles + 1));
     // N-sized arrays hold `C` agents: the rods of a cycle grow up to max_agents
     const uint64_t C = (is_rod(ctx) && ctx->cycle_on) ? std::max<uint64_t>(N, ctx->cyc.max_agents) : N;
     ctx->cap_agents = C;

@@ -12,7 +12,7 @@
 //   k_gather_integrate_point  arrivals put in order of previous slot,   } previous slot (sort_cells_in_voxels,
 //                      the full mechanics update written into the       }  update_mechanics.rs:418-513)
 //                      agent's new sorted slot, and the force records
-//   (set-up sorts and rods order the arrivals with k_fixup; systems whose voxels
+//   (set-up sorts order the arrivals with k_fixup; systems whose voxels
 //   fit one scan tile run k_sort_small, the scans and the scatter in one workgroup)
 //
 // Agents live in SoA arrays sorted by voxel; a voxel's agents are the slots
@@ -51,7 +51,7 @@ struct Arrays {
     Control* ctrl;
     uint32_t* start;  // [Vt + 1]
     uint32_t* start_local;  // [Vt] offset of each voxel inside its scan tile (k_scan_local)
-    uint32_t* tile_off;     // [n_tiles] offset of each scan tile (k_scan_tiles)
+    uint32_t* tile_off;     // [n_tiles + 1] sum of each scan tile (k_scan_local), or its offset (k_scan_tiles)
     uint32_t* count;  // [Vt] arrivals per next voxel (atomic ranks)
     uint32_t* stay;   // [Vt] agents binned ahead that stay in their voxel (zero otherwise)
     uint32_t* key;    // [N] next voxel
@@ -87,7 +87,7 @@ __device__ __forceinline__ void raise_error(Control* c, uint32_t kind, uint64_t 
 
 // An earlier step than t raised an error.  The kernels of the steps after a
 // failing one do nothing (the ones before the sort check this, the ones after it
-// read Control::skip, set by k_scan_tiles), so the state stays at the end of the
+// read Control::skip, set by k_scan_local), so the state stays at the end of the
 // failing step, where run_simulation! returns the error (run_sim.rs:380-403).
 __device__ __forceinline__ bool halted(const Control* c, uint64_t t) {
     return c->error_flags != 0 && (c->error_key >> 32) < t;
@@ -1388,8 +1388,11 @@ constexpr int kScanTile = kBlock * kScanItems;
 __global__ __launch_bounds__(kBlock) void k_scan_local(uint32_t* __restrict__ count,
                                                         const uint32_t* __restrict__ stay,
                                                         uint32_t* __restrict__ start_local, uint32_t* __restrict__ bsum,
-                                                        uint32_t Vt, const Control* ctrl) {
-    if (halted(ctrl, ctrl->step)) return;
+                                                        uint32_t Vt, Control* ctrl) {
+    const bool skip = halted(ctrl, ctrl->step);
+    // for the sort's later kernels (no block of this one reads it)
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->skip = skip ? 1u : 0u;
+    if (skip) return;
     static_assert(kScanItems == 8, "two uint4 per group");
     const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
     const bool whole = base + kScanItems <= Vt;
@@ -1439,16 +1442,11 @@ __global__ __launch_bounds__(kBlock) void k_scan_local(uint32_t* __restrict__ co
     if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-// Single block: exclusive scan of the tile sums in place (the tile offsets);
-// start[Vt] = total.  advance != 0 also completes the step counter (every kernel
-// that reads it for this step has run; the gather reads the new value).
+// Single block: exclusive scan of the tile sums in place (the tile offsets), for
+// grids of more than kScatterTiles scan tiles.
 __global__ __launch_bounds__(kBlock) void k_scan_tiles(uint32_t* __restrict__ bsum, uint32_t n_tiles,
-                                                        uint32_t* __restrict__ start, uint32_t Vt, Control* ctrl,
-                                                        uint32_t advance) {
-    const bool skip = halted(ctrl, ctrl->step);
-    __syncthreads();  // every thread has read the control block before thread 0 writes it
-    if (threadIdx.x == 0) ctrl->skip = skip ? 1u : 0u;
-    if (skip) return;
+                                                        const Control* ctrl) {
+    if (ctrl->skip) return;
     uint32_t carry = 0;
     for (uint32_t base = 0; base < n_tiles; base += kBlock) {
         uint32_t q = base + threadIdx.x;
@@ -1458,24 +1456,46 @@ __global__ __launch_bounds__(kBlock) void k_scan_tiles(uint32_t* __restrict__ bs
         if (q < n_tiles) bsum[q] = carry + ex;
         carry += total;
     }
-    if (threadIdx.x == 0) {
-        start[Vt] = carry;
-        if (advance) ctrl->step += 1;
-    }
+    if (threadIdx.x == 0) bsum[n_tiles] = carry;
 }
 
 // Thread g writes the final start of voxel g (tile-local offset + tile offset) and
 // places agent g in the slot list of its next voxel: a stayer at its rank, an
 // arrival (kMoved) after the voxel's stayers in atomic order.  Launched over
-// max(N, Vt) threads.
-__global__ __launch_bounds__(kBlock) void k_scatter(Arrays A) {
+// max(N, Vt) threads.  Thread 0 writes start[Vt]; advance != 0 also completes the
+// step counter (every kernel that reads it for this step has run; the gather reads
+// the new value).
+// SCAN: every workgroup scans the tile sums itself (two per thread): one more dependent
+// load and two barriers in place of k_scan_tiles, a 4.5 us launch in a chain of small
+// kernels.  The scatter stays at 4.7 us for 30,000 and 4.9 for 300,000 agents (a
+// 30,000-agent step 32.5 -> 28.9 us) and goes from 6.0 to 7.5 for 1M in 432 tiles; with
+// 1728 tiles per workgroup the step lost 1.7 %, hence the line at two per thread.
+constexpr uint32_t kScatterTiles = 512;
+template <bool SCAN>
+__global__ __launch_bounds__(kBlock) void k_scatter(Arrays A, uint32_t n_tiles, uint32_t advance) {
     if (A.ctrl->skip) return;
+    __shared__ uint32_t s_off[SCAN ? kScatterTiles : 1];
+    uint32_t total = 0;
+    const uint32_t* off = A.tile_off;
+    if constexpr (SCAN) {
+        const uint32_t q = 2u * threadIdx.x;
+        const uint32_t x = q < n_tiles ? A.tile_off[q] : 0u, y = q + 1u < n_tiles ? A.tile_off[q + 1u] : 0u;
+        const uint32_t ex = block_exclusive_scan(x + y, total);
+        s_off[q] = ex;
+        s_off[q + 1u] = ex + x;
+        __syncthreads();
+        off = s_off;
+    }
     const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (g < A.Vt) A.start[g] = A.start_local[g] + A.tile_off[g / kScanTile];
+    if (g == 0) {
+        A.start[A.Vt] = SCAN ? total : A.tile_off[n_tiles];
+        if (advance) A.ctrl->step += 1;
+    }
+    if (g < A.Vt) A.start[g] = A.start_local[g] + off[g / kScanTile];
     if (g >= A.N) return;
     const uint32_t k = A.key[g], r = A.rank[g];
     const uint32_t pos = (r & kMoved) ? A.stay[k] + (r & ~kMoved) : r;
-    A.perm[A.start_local[k] + A.tile_off[k / kScanTile] + pos] = (uint32_t)g;
+    A.perm[A.start_local[k] + off[k / kScanTile] + pos] = (uint32_t)g;
 }
 
 // Small systems (every voxel in one scan tile, at most kSmallSortAgents agents):
@@ -1626,19 +1646,23 @@ __device__ __forceinline__ void bin_ahead(const Arrays& A, const InstParams& P, 
 // voxel v of the current order: the agents of v that stay get consecutive ranks
 // in slot order and their number goes to stay[v]; the others take an atomic rank
 // among the arrivals of their next voxel (count), flagged with kMoved, which the
-// scatter places after that voxel's stayers; k_fixup puts the arrivals in order.
-__global__ __launch_bounds__(kBlock) void k_rank_ahead(Arrays A) {
-    if (halted(A.ctrl, A.ctrl->step)) return;
-    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (v >= A.Vt) return;
+// scatter places after that voxel's stayers; k_fixup (set-up sorts) or the gather
+// puts the arrivals in order.
+__device__ __forceinline__ void rank_voxel(const Arrays& A, uint32_t v) {
     const uint32_t b = A.start[v], e = A.start[v + 1];
     uint32_t n = 0;
     for (uint32_t s = b; s < e; s++) {
         const uint32_t k = A.key[s];
-        if (k == (uint32_t)v) A.rank[s] = n++;
+        if (k == v) A.rank[s] = n++;
         else A.rank[s] = kMoved | atomicAdd(&A.count[k], 1u);
     }
     A.stay[v] = n;
+}
+
+__global__ __launch_bounds__(kBlock) void k_rank_ahead(Arrays A) {
+    if (halted(A.ctrl, A.ctrl->step)) return;
+    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (v < A.Vt) rank_voxel(A, (uint32_t)v);
 }
 
 // Permutes the state into sorted order and writes the force records, without
@@ -1691,7 +1715,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_point(Arrays A, StateBuf src,
 // slot s (i itself, or arrival_slot's place among the voxel's arrivals); its
 // update (the same point_step as in k_key_point, so the same position) is computed
 // here and the new state written straight to slot s, together with the force
-// record for the next step.  k_scan_tiles has already advanced the step counter,
+// record for the next step.  The scatter has already advanced the step counter,
 // so this step started after step - 1 steps.
 template <int D, bool MIXED, int MECH>
 __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, StateBuf src, StateBuf dst,

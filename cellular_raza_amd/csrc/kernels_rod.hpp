@@ -8,7 +8,7 @@
 //                            pair weights (update_mechanics.rs:178-220)
 //   k_key_rod                next vertex positions, per-vertex reflection
 //                            (bacterial_rods.rs:489-533), centroid voxel + rank
-//   k_scan_local/tiles, k_scatter, k_fixup   as for point agents (slots are rods)
+//   k_scan_local/tiles, k_scatter   as for point agents (slots are rods)
 //   k_gather_integrate_rod   RodMechanics::calculate_increment (bacterial_rods.rs:157-240)
 //                            + solver, written into the rod's new slot
 // State arrays are the point arrays with K = nv * dim components per slot; the
@@ -68,7 +68,7 @@ __device__ __forceinline__ bool rod_lane(const BlockWork& w, uint32_t nv, uint64
 constexpr uint32_t kRodLdsBytes = 36 * 1024;
 template <int D, int POT, bool MIXED>
 __global__ __launch_bounds__(kBlock, 4) void k_force_rod(Arrays A, StateBuf S, RodArgs R, uint32_t physical,
-                                                          uint32_t no_lds) {
+                                                          uint32_t no_lds, uint32_t rank) {
     if (halted(A.ctrl, A.ctrl->step)) return;
     const BlockWork w = A.work[blockIdx.x];
     uint64_t s;
@@ -151,9 +151,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_force_rod(Arrays A, StateBuf S, R
         }
     }
     __syncthreads();
-    if (!active) return;
     // this lane's own row among the block's (0 or 1)
-    const uint32_t orow = ((S.vox[s] - voff) / n2) == s_row[0] ? 0u : 1u;
+    const uint32_t orow = !active || ((S.vox[s] - voff) / n2) == s_row[0] ? 0u : 1u;
     auto work = [&](auto stg) {
         constexpr bool STG = decltype(stg)::value;
         auto bnd_of = [&](uint32_t j, int32_t base) -> double4 {
@@ -559,8 +558,17 @@ __global__ __launch_bounds__(kBlock, 4) void k_force_rod(Arrays A, StateBuf S, R
         A.sense[s * nv + v] = n;
     }
     };
-    if (staged) work(std::true_type{});
-    else work(std::false_type{});
+    if (active) {
+        if (staged) work(std::true_type{});
+        else work(std::false_type{});
+    }
+    // the step's re-binning ranks (k_rank_ahead's work: keys binned ahead, which the
+    // forces do not read), a share of the voxels per workgroup; each wave comes here
+    // after its own forces (ahead of them the ranks' loads delayed every workgroup:
+    // 200,000 rods 326 -> 357 us)
+    if (rank)
+        for (uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x; g < A.Vt; g += (uint64_t)gridDim.x * kBlock)
+            rank_voxel(A, (uint32_t)g);
 }
 
 // Normal k of a rod's K normals for (agent, step): Philox block k / 2, element k % 2.
@@ -854,7 +862,7 @@ __device__ __forceinline__ void rod_ahead(const InstParams& P, const StepArgs& s
 }
 
 // Gather + integrate for rods: lane (s, v) computes vertex row v of the rod that
-// lands in sorted slot s (coming from slot o = perm[s]).  With AHEAD it also bins
+// lands in sorted slot s (coming from slot o).  With AHEAD it also bins
 // the rod for the next step, as k_key_rod would after that step's forces: the
 // position update needs neither the force nor noise other than the next step's
 // (Philox, or none), so the new vertex positions, velocities and ring give the
@@ -874,16 +882,25 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
     // streams read or written once (forces, the new state and ring) bypass the
     // caches' retention (nontemporal; 200,000 2-D rods 125 -> 118 us); positions stay cached, the
     // neighbouring vertex rows read them again.
+    // The rods of a step come in the order of k_scatter: an arrival's sorted slot is
+    // arrival_slot's (looked up once per rod).
+    __shared__ uint32_t s_src[kBlock], s_dst[kBlock];
+    if (threadIdx.x < w.count) {
+        const uint32_t i = (uint32_t)w.first + threadIdx.x, o = A.perm[i];
+        s_src[threadIdx.x] = o;
+        s_dst[threadIdx.x] = INTEGRATE ? arrival_slot(A, i, o, A.key[o]) : i;
+    }
+    __syncthreads();
     const uint32_t rr = threadIdx.x % R.rpb, v = threadIdx.x / R.rpb;
-    const uint64_t s = w.first + rr;
     const bool active = v < nv && rr < w.count;
+    const uint32_t o = active ? s_src[rr] : 0u;
+    const uint64_t s = active ? s_dst[rr] : 0u;
     const uint32_t lt = rr * nv + v;
     const InstParams& P = A.ip[w.inst];
     const uint64_t N = A.N;
     double nx[D], nvel[D];
     if constexpr (INTEGRATE) {  // bending window v of the rod, shared with the next two lanes
         if (active && v + 2 < nv) {
-            const uint32_t o = A.perm[s];
             auto pos = [&](int i, int k) { return src.pos[(uint64_t)(i * D + k) * N + o]; };
             double F[D];
             rod_bend_window<D>(P, pos, (int)v, F);
@@ -893,7 +910,6 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
         __syncthreads();
     }
     if (active) {
-        const uint32_t o = A.perm[s];
         const uint32_t id = src.id[o];
         if (INTEGRATE) {
             const uint64_t t = A.ctrl->step - 1;
@@ -976,11 +992,11 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
         }
     }
     __syncthreads();
-    // the force records rec[slot][K] of the block's rods, a contiguous range,
-    // written element by element from LDS
+    // the force records rec[slot][K] of the block's rods, a contiguous range but for
+    // arrivals, written element by element from LDS
     for (uint32_t e = threadIdx.x; e < w.count * K; e += kBlock) {
         const uint32_t r = e / K, c = e - r * K, vq = c / D;
-        R.rec[w.first * K + e] = newpos[(r * nv + vq) * 3 + (c - vq * D)];
+        R.rec[(uint64_t)s_dst[r] * K + c] = newpos[(r * nv + vq) * 3 + (c - vq * D)];
     }
     // the rod's vertex mean (every lane of the rod computes the same)
     auto mean = [&](double* c) {
