@@ -198,6 +198,8 @@ constexpr uint32_t kNoAllocMaxInstances = 1u << 16;
 constexpr size_t kNoAllocScanReserve = (size_t)1 << 20;
 // Steps per long graph replay (even, so that a replay keeps the buffer parity).
 constexpr uint32_t kLongGraphSteps = 16;
+// Steps of a call from which the carry of the older ring entry is left to the last one.
+constexpr uint32_t kCarryLastSteps = 8;
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kNoAllocScratchBytes = align256(kNoAllocMaxAgents) + 4 * align256(4 * (kNoAllocMaxAgents + 1)) +
                                         align256(4 * (size_t)kNoAllocMaxInstances) + kNoAllocScanReserve;
@@ -2207,6 +2209,11 @@ crm_status crm_step(crm_ctx* ctx, uint32_t n_steps, const double* noise) {
             }
         ctx->graphs_stale = false;
     }
+    // (short calls write the whole ring in every step: the launch costs them more)
+    if (ctx->cfg.solver_order == 2 && n_steps >= kCarryLastSteps) {
+        hipLaunchKernelGGL(k_set_last_step, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl, ctx->step + n_steps - 1);
+        CRM_HIP(hipGetLastError());
+    }
     uint32_t s = 0;
     if (graphs) {  // each graph launch costs the device a few microseconds
         while (s + kLongGraphSteps <= n_steps) {
@@ -2231,6 +2238,16 @@ crm_status crm_step(crm_ctx* ctx, uint32_t n_steps, const double* noise) {
         if (t_err >= ctx->step && t_err < ctx->step + n_steps) {
             done = t_err + 1 - ctx->step;
             if ((n_steps - done) & 1) ctx->cur = 1 - ctx->cur;
+            if (done < n_steps && ctx->cfg.solver_order == 2) {
+                const StateBuf dst = ctx->buf[ctx->cur], src = ctx->buf[1 - ctx->cur];
+                ctx->cur = 1 - ctx->cur;  // the failing step's keys
+                const Arrays A = arrays(ctx);
+                ctx->cur = 1 - ctx->cur;
+                hipLaunchKernelGGL(k_carry_ring, dim3((uint32_t)((ctx->N + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                                   ctx->stream, A, src, dst, t_err, ctx->K);
+                CRM_HIP(hipGetLastError());
+                CRM_HIP(hipStreamSynchronize(ctx->stream));
+            }
         }
     }
     ctx->step += done;

@@ -1767,11 +1767,15 @@ __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, Sta
         __builtin_nontemporal_store(nx[k], &dst.pos[k * N + s]);
         __builtin_nontemporal_store(nv[k], &dst.vel[k * N + s]);
     }
-    // ring: the slot written this step gets (dx, dv), the other slot is carried over
+    // ring: the slot written this step gets (dx, dv).  The other slot's entry, which
+    // the next step overwrites before it reads the ring, is carried over by the last
+    // step of a call only (48 of 332 bytes per 3-D agent; a call that ends early at
+    // an error gets it from k_carry_ring)
     if (rg.cap > 0) {
+        const bool both = n_old > 0 && t >= A.ctrl->last_step;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const bool keep = (uint32_t)h < rg.cap && ((uint32_t)h == rg.wslot || n_old > 0);
+            const bool keep = (uint32_t)h < rg.cap && ((uint32_t)h == rg.wslot || both);
 #pragma unroll
             for (int k = 0; k < D; k++) {
                 if (h == (int)rg.wslot) {
@@ -1794,6 +1798,25 @@ __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, Sta
     if (dst.birth) dst.birth[s] = (uint32_t)birth;
     if constexpr (MECH != CRM_MECHANICS_BROWNIAN)
         bin_ahead<D, MECH>(A, P, sa, t + 1, id, s, nx, nv, hx[0], hx[1], key, birth);
+}
+
+// Index of the last step of the call that is about to run.
+__global__ void k_set_last_step(Control* c, uint64_t t) { c->last_step = t; }
+
+// After a call that ended at an error before its last step t: the older ring entry of
+// every agent, from the failing step's source buffer (the sort's arrays still hold that
+// step's order) to its destination.  K components per agent.
+__global__ __launch_bounds__(kBlock) void k_carry_ring(Arrays A, StateBuf src, StateBuf dst, uint64_t t, uint32_t K) {
+    const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= A.N) return;
+    const uint32_t o = A.perm[i];
+    const uint64_t s = arrival_slot(A, (uint32_t)i, o, A.key[o]);
+    if (t <= (src.birth ? src.birth[o] : 0u)) return;  // no older entry
+    const uint64_t h = 1u - (t & 1u);
+    for (uint32_t k = 0; k < K; k++) {
+        dst.hdx[(h * K + k) * A.N + s] = src.hdx[(h * K + k) * A.N + o];
+        dst.hdv[(h * K + k) * A.N + s] = src.hdv[(h * K + k) * A.N + o];
+    }
 }
 
 }  // namespace crm

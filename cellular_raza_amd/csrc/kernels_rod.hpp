@@ -944,7 +944,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
             }
             if (rg.cap > 0) {
                 const uint32_t n_hist = (uint32_t)min<uint64_t>(t + 1, rg.cap);
+                const bool both = t >= A.ctrl->last_step;  // (see k_gather_integrate_point)
                 for (uint32_t h = 0; h < n_hist; h++) {
+                    if (h != rg.wslot && !both) continue;
 #pragma unroll
                     for (int k = 0; k < D; k++) {
                         const uint64_t e = ((uint64_t)h * K + v * D + k) * N;

@@ -83,6 +83,9 @@ struct Control {
     uint64_t out_of_grid;   // agents that kept their voxel because the new index had no voxel
     uint32_t skip;          // set by k_scan_local / k_sort_small: this step's sort is skipped (an earlier step failed)
     uint32_t pad;
+    // index of the last step of the running crm_step call (or any earlier one): the
+    // steps before it leave the ring entry that no later step reads unwritten
+    uint64_t last_step;
 };
 
 }  // namespace crm
