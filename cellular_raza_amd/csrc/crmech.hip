@@ -219,6 +219,7 @@ struct crm_ctx {
     uint64_t Vt = 0;
     uint32_t pot_kind = 0, mech_kind = 0;
     bool symmetric = true;
+    bool wide_voxels = false;  // an instance's voxels are wider than kWideVoxels cutoffs
     bool mie_pow = false;  // an instance's Mie exponents are not integers
     std::string err;
 
@@ -517,7 +518,8 @@ crm_status launch_force_dpm(crm_ctx* ctx, StateBuf S, uint32_t rank) {
 // rank != 0: the force kernel also ranks the step's re-binning (keys binned ahead).
 template <int D, int POT>
 crm_status launch_force_dp(crm_ctx* ctx, StateBuf S, uint32_t rank) {
-    return ctx->lanes_log2 ? launch_force_dpm<D, POT, true>(ctx, S, rank) : launch_force_dpm<D, POT, false>(ctx, S, rank);
+    return ctx->lanes_log2 || ctx->wide_voxels ? launch_force_dpm<D, POT, true>(ctx, S, rank)
+                                               : launch_force_dpm<D, POT, false>(ctx, S, rank);
 }
 
 template <int D>
@@ -1727,6 +1729,7 @@ crm_status insert_agents_impl(crm_ctx* ctx, uint64_t n, const uint64_t* mother, 
         }
     };
     // the voxel a divided agent moves to (its list's voxel g if its position has none)
+    uint64_t kept = 0;  // agents of no voxel
     auto voxel_key = [&](const InstParams& P, const double* x, uint64_t g) -> uint32_t {
         uint32_t idx[3] = {0, 0, 0};
         bool ok = true;
@@ -1734,6 +1737,7 @@ crm_status insert_agents_impl(crm_ctx* ctx, uint64_t n, const uint64_t* mother, 
             const uint32_t ax = k + 3 - D;
             ok = ok && axis_index_host(x[k], P.min[ax], P.dx[ax], P.n[ax], idx[ax]);
         }
+        kept += ok ? 0u : 1u;
         return ok ? (uint32_t)(P.voxel_offset + ((uint64_t)idx[0] * P.n[1] + idx[1]) * P.n[2] + idx[2])
                   : (uint32_t)g;
     };
@@ -1807,6 +1811,10 @@ crm_status insert_agents_impl(crm_ctx* ctx, uint64_t n, const uint64_t* mother, 
                            ctx->stream));
     CRM_HIP(hipMemcpyAsync(ctx->d_key, key2.data(), N2 * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
     CRM_TRY(rebuild_work(ctx));
+    if (kept) {
+        hipLaunchKernelGGL(k_note_out_of_grid, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl, kept);
+        CRM_HIP(hipGetLastError());
+    }
     {
         std::vector<ForceTile> tiles;  // the tile shape follows the density
         make_tiles(ctx, ctx->policy, tiles);
@@ -1924,6 +1932,8 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
         }
         fill_pot<double>(P.pd, I.potential);
         fill_pot<float>(P.pf, I.potential);
+        const double rc = I.potential.kind == CRM_POTENTIAL_CELL_SORTING ? P.pd.rel_range * P.pd.two_radius : P.pd.cutoff;
+        if (std::fmin(P.dx[1], P.dx[2]) > kWideVoxels * rc) ctx->wide_voxels = true;
         if (I.potential.kind == CRM_POTENTIAL_MIE && (P.pd.ien1 < 0 || P.pd.iem1 < 0)) ctx->mie_pow = true;
         const crm_mechanics& M = I.mechanics;
         P.mass = M.mass;

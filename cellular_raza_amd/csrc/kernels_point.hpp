@@ -742,6 +742,7 @@ constexpr int kTileRowsMax = 29;
 constexpr int kLdsVoxelStarts = 768;    // 1.5 KiB of voxel-start indices (staged voxels + 1)
 constexpr int kOwnVoxMax = 256;         // own voxels per tile
 constexpr int kSortBins = 64;           // candidate-count classes for the lane order
+constexpr double kWideVoxels = 1.25;    // voxel edges per cutoff above which streams are cut to the cutoff's reach
 
 struct ForceTile {
     uint32_t inst, a0, b0, b1, c0, c1;
@@ -796,8 +797,9 @@ __device__ __forceinline__ uint32_t small_div(uint32_t a, float inv_d) {
 // starts) in LDS, then one lane per own agent sums its forces from LDS.  A tile
 // whose region does not fit (local crowding) reads global memory instead; the
 // candidate order and the arithmetic are the same.
-// MULTI: the tiling policy gives each agent 2^lanes_log2 lanes (a separate
-// instantiation, so that the one-lane kernel carries none of the group logic).
+// MULTI: the tiling policy gives each agent 2^lanes_log2 lanes, or the voxels are wide
+// (a separate instantiation, so that the common one-lane kernel carries none of the
+// group and reach logic).
 template <int D, int POT, bool MIXED, bool SENSE, bool MULTI>
 __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A, StateBuf S,
                                                                      const ForceTile* __restrict__ tiles,
@@ -973,6 +975,48 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
             const uint32_t n_own = own_pre[n_ownv];
             LdsSource<D, MIXED> src{lds, lsp, vst, G, NP, n_vox, A.start, voff, n1, n2, lsub};
             const float inv_w = 1.0f / (float)W;
+            // Squared distances of an own agent to the borders of its voxel: to the rows
+            // before and after it and to the columns.  What lies behind a border
+            // farther than the cutoff (lim2 has 1e-5 to spare for the float arithmetic)
+            // is left out of the stream: no candidate there is ever marked, so the
+            // sums are the same.  With voxels of twice the cutoff that is more than half
+            // of the candidates (1600 crowded 3-D agents: 28 -> 21 us); with voxels as
+            // wide as the cutoff it is the corner pillars, 9.5 %, but a wave's longest
+            // streams stay, and the code alone costs the one-lane kernels their last
+            // registers (4M-agent lattice 501 -> 512 us): it is part of the MULTI kernels,
+            // which serve every context with voxels wider than 1.25 cutoffs, and idle
+            // below that.  Agents may be outside their voxel only after a position
+            // without one (out_of_grid) or a failed step: then nothing is left out.
+            struct Reach {
+                float up2 = 0.0f, down2 = 0.0f, lo2 = 0.0f, hi2 = 0.0f;
+            };
+            const double rcut = cut_radius<POT, double>(P.pd);
+            const bool trim = MULTI && !SENSE && fmin(P.dx[1], P.dx[2]) > kWideVoxels * rcut &&
+                              A.ctrl->out_of_grid == 0 && A.ctrl->error_flags == 0;
+            const float lim2 = (float)(rcut * rcut * (1.0 + 1e-5));
+            auto reach_of = [&](const Rec& me, uint32_t r, uint32_t c) {  // own row r, column c
+                float lo[2], hi[2];                                       // row, column
+                if constexpr (MIXED) {
+                    const int one = 1 << G.bits;
+                    const int q[2] = {(D == 3 ? me.y : me.x) - ((int)(r + 1) << G.bits),
+                                      (D == 3 ? me.z : me.y) - ((int)(c - G.cl) << G.bits)};
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                        lo[k] = (float)q[k] * unit[D - 2 + k];
+                        hi[k] = (float)(one - q[k]) * unit[D - 2 + k];
+                    }
+                } else {
+                    const double x[2] = {D == 3 ? me.y : me.x, D == 3 ? me.z : me.y};
+                    const uint32_t i[2] = {T.b0 + r, c};
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                        const double f = x[k] - (P.min[1 + k] + (double)i[k] * P.dx[1 + k]);
+                        lo[k] = fmaxf((float)f, 0.0f);  // (a border's rounding may put it outside)
+                        hi[k] = fmaxf((float)(P.dx[1 + k] - f), 0.0f);
+                    }
+                }
+                return Reach{lo[0] * lo[0], hi[0] * hi[0], lo[1] * lo[1], hi[1] * hi[1]};
+            };
             // own agent t: own voxel u (largest u with own_pre[u] <= t), LDS index,
             // global slot, and the three ranges of its stream
             auto own_agent = [&](uint32_t t, uint32_t& self, Span& ov, Walk3& w) -> uint32_t {
@@ -987,15 +1031,20 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                 const uint32_t vo = src.vox(r + 1, c, PA_OWN);
                 self = (uint32_t)vst[vo] + k;
                 ov = Span{vst[vo], vst[vo + 1]};
-                const uint32_t c_lo = c == 0 ? 0 : c - 1, c_hi = min(c + 2, n2);
                 // stencil rows r, r + 1, r + 2 of the region (b - 1, b, b + 1; rows
-                // outside the grid are staged empty)
-                w.j = vst[src.vox(r, c_lo, 0)];
-                w.je = vst[src.vox(r, c_hi, 0)];
-                w.j1 = vst[src.vox(r + 1, c_lo, 0)];
-                w.e1 = vst[src.vox(r + 1, c_hi, 0)];
-                w.j2 = vst[src.vox(r + 2, c_lo, 0)];
-                w.e2 = vst[src.vox(r + 2, c_hi, 0)];
+                // outside the grid are staged empty), each from its first to its last
+                // column that the cutoff reaches
+                Reach h;
+                if (MULTI && trim) h = reach_of(Recs::at(lds, self * Recs::kBytes), r, c);
+                auto range = [&](uint32_t q, float row2, uint32_t& j, uint32_t& je) {
+                    const uint32_t cl = c - (c > 0u && !(row2 + h.lo2 > lim2) ? 1u : 0u);
+                    const uint32_t ch = c + 1u + (c + 1u < n2 && !(row2 + h.hi2 > lim2) ? 1u : 0u);
+                    j = vst[src.vox(r + q, cl, 0)];
+                    je = vst[src.vox(r + q, row2 > lim2 ? cl : ch, 0)];
+                };
+                range(0, h.up2, w.j, w.je);
+                range(1, 0.0f, w.j1, w.e1);
+                range(2, h.down2, w.j2, w.e2);
                 w.left = 2;
                 return own_gs[lo] + k;
             };
@@ -1799,6 +1848,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, Sta
     if constexpr (MECH != CRM_MECHANICS_BROWNIAN)
         bin_ahead<D, MECH>(A, P, sa, t + 1, id, s, nx, nv, hx[0], hx[1], key, birth);
 }
+
+// Agents that were put in a voxel their position is not in (inserted ones).
+__global__ void k_note_out_of_grid(Control* c, uint64_t n) { c->out_of_grid += n; }
 
 // Index of the last step of the call that is about to run.
 __global__ void k_set_last_step(Control* c, uint64_t t) { c->last_step = t; }
