@@ -240,11 +240,12 @@ struct crm_ctx {
     std::vector<uint32_t> tile_rows, tile_cols, tile_count;  // per instance
     Control* d_ctrl = nullptr;
     uint32_t* d_start = nullptr;
-    uint32_t* d_count = nullptr;
+    uint32_t* d_count = nullptr;        // per voxel: arrivals, stayers, list heads of two steps by parity, delta
     uint32_t* d_start_local = nullptr;  // [Vt] voxel offsets inside their scan tile
     uint32_t* d_bsum = nullptr;         // [n_tiles + 1] scan tile sums, then (more than kScatterTiles) offsets, total
     uint32_t n_tiles = 0;
-    uint32_t* d_key = nullptr;
+    uint32_t n_scan = 0, scan_shift = 0;  // a step's scan tiles (Arrays)
+    uint32_t* d_key = nullptr;          // [2][N] keys by state-buffer parity, then (2 cap_agents in) list links
     uint32_t* d_rank = nullptr;
     uint32_t* d_perm = nullptr;
     double* d_force = nullptr;
@@ -398,8 +399,8 @@ void free_device(crm_ctx* ctx) {
     ctx->noise_cap = 0;
 }
 
-// d_count holds the arrivals per voxel, then (from this offset, 256-byte aligned)
-// the stayers per voxel.
+// d_count holds five sections of this many voxels (256-byte aligned): arrivals and
+// stayers of set-up sorts, and a step's list heads (two) and deltas.
 uint64_t stay_offset(const crm_ctx* ctx) { return (ctx->Vt + 63) & ~(uint64_t)63; }
 
 bool force_f32(const crm_ctx* ctx);
@@ -414,12 +415,20 @@ Arrays arrays(crm_ctx* ctx) {
     A.tile_off = ctx->d_bsum;
     A.count = ctx->d_count;
     A.stay = ctx->d_count + stay_offset(ctx);
-    // two key buffers: the current step's (read by the sort) and the next step's
-    // (binned ahead by the gather), by state-buffer parity
+    // two buffers of keys, list heads and links: the current step's (read by the scan and
+    // the gather) and the next step's (binned ahead by the gather), by state-buffer parity
     A.key = ctx->d_key + (size_t)ctx->cur * ctx->N;
     A.rank = ctx->d_rank;
     A.key_next = ctx->d_key + (size_t)(1 - ctx->cur) * ctx->N;
     A.perm = ctx->d_perm;
+    const uint64_t Vs = stay_offset(ctx);
+    A.head = ctx->d_count + (2 + (size_t)ctx->cur) * Vs;
+    A.head_next = ctx->d_count + (3 - (size_t)ctx->cur) * Vs;
+    A.delta = reinterpret_cast<int32_t*>(ctx->d_count + 4 * Vs);
+    A.link = ctx->d_key + 2 * ctx->cap_agents + (size_t)ctx->cur * ctx->N;
+    A.link_next = ctx->d_key + 2 * ctx->cap_agents + (size_t)(1 - ctx->cur) * ctx->N;
+    A.n_scan = ctx->n_scan;
+    A.scan_shift = ctx->scan_shift;
     A.force = ctx->d_force;
     A.forcef = force_f32(ctx) ? reinterpret_cast<float*>(ctx->d_force) : nullptr;
     A.rec64 = ctx->d_rec64;
@@ -491,57 +500,57 @@ crm_status t_end(crm_ctx* ctx, int cls) {
     } while (0)
 
 template <int D, int POT, bool MULTI>
-crm_status launch_force_dpm(crm_ctx* ctx, StateBuf S, uint32_t rank) {
+crm_status launch_force_dpm(crm_ctx* ctx, StateBuf S, uint32_t n_scan) {
     Arrays A = arrays(ctx);
     const uint32_t phys = ctx->cfg.weighting == CRM_WEIGHT_PHYSICAL;
     const uint32_t sym = ctx->symmetric;
     const uint32_t no_lds = (ctx->cfg.flags & CRM_FLAG_NO_LDS) ? 1u : 0u;
-    const dim3 g(ctx->n_force_tiles), b(kBlock);
+    const dim3 g(ctx->n_force_tiles + n_scan), b(kBlock);
     const uint32_t lg = ctx->lanes_log2;
     // sensing has kernels of its own, so the force-only kernels carry none of it
     const bool mixed = ctx->cfg.precision == CRM_PRECISION_MIXED, sense = A.sense != nullptr;
     if (mixed && sense)
         hipLaunchKernelGGL((k_force_tiled<D, POT, true, true, MULTI>), g, b, 0, ctx->stream, A, S, ctx->d_tiles, phys,
-                           sym, no_lds, rank, lg);
+                           sym, no_lds, n_scan, lg);
     else if (mixed)
         hipLaunchKernelGGL((k_force_tiled<D, POT, true, false, MULTI>), g, b, 0, ctx->stream, A, S, ctx->d_tiles, phys,
-                           sym, no_lds, rank, lg);
+                           sym, no_lds, n_scan, lg);
     else if (sense)
         hipLaunchKernelGGL((k_force_tiled<D, POT, false, true, MULTI>), g, b, 0, ctx->stream, A, S, ctx->d_tiles, phys,
-                           sym, no_lds, rank, lg);
+                           sym, no_lds, n_scan, lg);
     else
         hipLaunchKernelGGL((k_force_tiled<D, POT, false, false, MULTI>), g, b, 0, ctx->stream, A, S, ctx->d_tiles,
-                           phys, sym, no_lds, rank, lg);
+                           phys, sym, no_lds, n_scan, lg);
     return CRM_OK;
 }
 
-// rank != 0: the force kernel also ranks the step's re-binning (keys binned ahead).
+// n_scan != 0: further workgroups of the force kernel scan the next order (scan_moves).
 template <int D, int POT>
-crm_status launch_force_dp(crm_ctx* ctx, StateBuf S, uint32_t rank) {
-    return ctx->lanes_log2 || ctx->wide_voxels ? launch_force_dpm<D, POT, true>(ctx, S, rank)
-                                               : launch_force_dpm<D, POT, false>(ctx, S, rank);
+crm_status launch_force_dp(crm_ctx* ctx, StateBuf S, uint32_t n_scan) {
+    return ctx->lanes_log2 || ctx->wide_voxels ? launch_force_dpm<D, POT, true>(ctx, S, n_scan)
+                                               : launch_force_dpm<D, POT, false>(ctx, S, n_scan);
 }
 
 template <int D>
-crm_status launch_force_d(crm_ctx* ctx, StateBuf S, uint32_t rank) {
+crm_status launch_force_d(crm_ctx* ctx, StateBuf S, uint32_t n_scan) {
     switch (ctx->pot_kind) {
-        case CRM_POTENTIAL_MORSE: return launch_force_dp<D, CRM_POTENTIAL_MORSE>(ctx, S, rank);
+        case CRM_POTENTIAL_MORSE: return launch_force_dp<D, CRM_POTENTIAL_MORSE>(ctx, S, n_scan);
         case CRM_POTENTIAL_MIE:
-            return ctx->mie_pow ? launch_force_dp<D, kPotentialMiePow>(ctx, S, rank)
-                                : launch_force_dp<D, CRM_POTENTIAL_MIE>(ctx, S, rank);
+            return ctx->mie_pow ? launch_force_dp<D, kPotentialMiePow>(ctx, S, n_scan)
+                                : launch_force_dp<D, CRM_POTENTIAL_MIE>(ctx, S, n_scan);
         case CRM_POTENTIAL_BOUND_LENNARD_JONES:
-            return launch_force_dp<D, CRM_POTENTIAL_BOUND_LENNARD_JONES>(ctx, S, rank);
-        case CRM_POTENTIAL_MORSE_SPECIES: return launch_force_dp<D, CRM_POTENTIAL_MORSE_SPECIES>(ctx, S, rank);
-        case CRM_POTENTIAL_CELL_SORTING: return launch_force_dp<D, CRM_POTENTIAL_CELL_SORTING>(ctx, S, rank);
-        case CRM_POTENTIAL_NONE: return launch_force_dp<D, CRM_POTENTIAL_NONE>(ctx, S, rank);
+            return launch_force_dp<D, CRM_POTENTIAL_BOUND_LENNARD_JONES>(ctx, S, n_scan);
+        case CRM_POTENTIAL_MORSE_SPECIES: return launch_force_dp<D, CRM_POTENTIAL_MORSE_SPECIES>(ctx, S, n_scan);
+        case CRM_POTENTIAL_CELL_SORTING: return launch_force_dp<D, CRM_POTENTIAL_CELL_SORTING>(ctx, S, n_scan);
+        case CRM_POTENTIAL_NONE: return launch_force_dp<D, CRM_POTENTIAL_NONE>(ctx, S, n_scan);
         case CRM_POTENTIAL_CELL_SORTING_LANGEVIN:
-            return launch_force_dp<D, CRM_POTENTIAL_CELL_SORTING_LANGEVIN>(ctx, S, rank);
+            return launch_force_dp<D, CRM_POTENTIAL_CELL_SORTING_LANGEVIN>(ctx, S, n_scan);
     }
     return CRM_INVALID_ARGUMENT;
 }
 
 template <int D, bool MIXED>
-crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S, uint32_t rank) {
+crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S, uint32_t n_scan) {
     Arrays A = arrays(ctx);
     const RodArgs R = rod_args(ctx);
     const uint32_t phys = ctx->cfg.weighting == CRM_WEIGHT_PHYSICAL;
@@ -549,42 +558,41 @@ crm_status launch_force_rod_dm(crm_ctx* ctx, StateBuf S, uint32_t rank) {
     const dim3 g(ctx->n_work), b(kBlock);
     switch (ctx->pot_kind) {
         case CRM_POTENTIAL_MORSE:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             return CRM_OK;
         case CRM_POTENTIAL_MORSE_SPECIES:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE_SPECIES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MORSE_SPECIES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             return CRM_OK;
         case CRM_POTENTIAL_MIE:
             if (ctx->mie_pow)
-                hipLaunchKernelGGL((k_force_rod<D, kPotentialMiePow, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+                hipLaunchKernelGGL((k_force_rod<D, kPotentialMiePow, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             else
-                hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+                hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_MIE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             return CRM_OK;
         case CRM_POTENTIAL_BOUND_LENNARD_JONES:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_BOUND_LENNARD_JONES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_BOUND_LENNARD_JONES, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             return CRM_OK;
         case CRM_POTENTIAL_NONE:
-            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_NONE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, rank);
+            hipLaunchKernelGGL((k_force_rod<D, CRM_POTENTIAL_NONE, MIXED>), g, b, 0, ctx->stream, A, S, R, phys, no_lds, n_scan);
             return CRM_OK;
     }
     return CRM_INVALID_ARGUMENT;
 }
 
 template <int D>
-crm_status launch_force_rod_d(crm_ctx* ctx, StateBuf S, uint32_t rank) {
-    return ctx->cfg.precision == CRM_PRECISION_MIXED ? launch_force_rod_dm<D, true>(ctx, S, rank)
-                                                     : launch_force_rod_dm<D, false>(ctx, S, rank);
+crm_status launch_force_rod_d(crm_ctx* ctx, StateBuf S, uint32_t n_scan) {
+    return ctx->cfg.precision == CRM_PRECISION_MIXED ? launch_force_rod_dm<D, true>(ctx, S, n_scan)
+                                                     : launch_force_rod_dm<D, false>(ctx, S, n_scan);
 }
 
-// rank: agents binned ahead -- the force kernel also ranks the step's
-// re-binning (only inside a step: a force evaluation on its own must leave the
-// histogram alone).
-crm_status launch_force(crm_ctx* ctx, bool rank = false) {
+// scan: agents binned ahead -- the force kernel also scans the step's next order
+// (only inside a step: a force evaluation on its own must leave the moves alone).
+crm_status launch_force(crm_ctx* ctx, bool scan = false) {
     CRM_TRY(t_begin(ctx));
     StateBuf S = ctx->buf[ctx->cur];
     ctx->sense_parity = ctx->cur;
     crm_status st;
-    const uint32_t r = rank ? 1u : 0u;
+    const uint32_t r = scan ? ctx->n_scan : 0u;
     if (is_rod(ctx)) st = ctx->D == 2 ? launch_force_rod_d<2>(ctx, S, r) : launch_force_rod_d<3>(ctx, S, r);
     else st = ctx->D == 2 ? launch_force_d<2>(ctx, S, r) : launch_force_d<3>(ctx, S, r);
     if (st) return st;
@@ -647,7 +655,7 @@ crm_status launch_key(crm_ctx* ctx, const StepArgs& sa) {
         st = ctx->D == 2 ? launch_key_d<2>(ctx, S, sa) : launch_key_d<3>(ctx, S, sa);
     }
     if (st) return st;
-    CRM_TRY(launch_rank(ctx));
+    CRM_HIP(hipGetLastError());
     return t_end(ctx, CRM_KERNEL_INTEGRATE);
 }
 
@@ -695,18 +703,33 @@ crm_status launch_gather_setup_d(crm_ctx* ctx, StateBuf src, StateBuf dst, const
 
 bool keys_ahead(const crm_ctx* ctx);
 
-// scan + scatter + fixup + gather: the counting sort that rebuilds the voxel
-// lists from d_key / d_rank / d_count and moves the state to the other buffer.
-crm_status launch_sort(crm_ctx* ctx, bool advance, const StepArgs* sa) {
+template <int D>
+void launch_gather_rod(crm_ctx* ctx, StateBuf src, StateBuf dst, bool integrate, const StepArgs& sa) {
+    Arrays A = arrays(ctx);
+    const RodArgs R = rod_args(ctx);
+    const dim3 g(ctx->n_work), b(kBlock);
+    if (keys_ahead(ctx)) {
+        if (integrate) hipLaunchKernelGGL((k_gather_rod<D, true, true>), g, b, 0, ctx->stream, A, src, dst, R, sa);
+        else hipLaunchKernelGGL((k_gather_rod<D, false, true>), g, b, 0, ctx->stream, A, src, dst, R, sa);
+    } else {
+        if (integrate) hipLaunchKernelGGL((k_gather_rod<D, true, false>), g, b, 0, ctx->stream, A, src, dst, R, sa);
+        else hipLaunchKernelGGL((k_gather_rod<D, false, false>), g, b, 0, ctx->stream, A, src, dst, R, sa);
+    }
+}
+
+// scan + scatter + fixup + gather: the counting sort of a set-up, which rebuilds the
+// voxel lists from d_key / d_rank / d_count and moves the state to the other buffer.
+crm_status launch_sort(crm_ctx* ctx, const StepArgs* sa, bool clear_moves) {
     Arrays A = arrays(ctx);
     const uint32_t Vt = (uint32_t)ctx->Vt;
+    if (clear_moves)  // the gather notes the first ones
+        CRM_HIP(hipMemsetAsync(ctx->d_count + 2 * stay_offset(ctx), 0, sizeof(uint32_t) * 3 * stay_offset(ctx), ctx->stream));
     if (ctx->n_tiles == 1 && ctx->N <= kSmallSortAgents) {  // one workgroup does all three (timed as scan)
         CRM_TRY(t_begin(ctx));
-        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kBlock), 0, ctx->stream, A, (uint32_t)(advance ? 1 : 0));
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kBlock), 0, ctx->stream, A);
         CRM_TRY(t_end(ctx, CRM_KERNEL_SCAN));
     } else {
         const bool scan = ctx->n_tiles <= kScatterTiles;  // the scatter scans the tile sums itself
-        const uint32_t adv = advance ? 1u : 0u;
         CRM_TRY(t_begin(ctx));
         hipLaunchKernelGGL(k_scan_local, dim3(ctx->n_tiles), dim3(kBlock), 0, ctx->stream, ctx->d_count,
                            ctx->d_count + stay_offset(ctx), ctx->d_start_local, ctx->d_bsum, Vt, ctx->d_ctrl);
@@ -717,51 +740,22 @@ crm_status launch_sort(crm_ctx* ctx, bool advance, const StepArgs* sa) {
         CRM_TRY(t_begin(ctx));
         const uint64_t n_scatter = std::max<uint64_t>(ctx->N, Vt);
         const dim3 g((uint32_t)((n_scatter + kBlock - 1) / kBlock));
-        if (scan) hipLaunchKernelGGL(k_scatter<true>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles, adv);
-        else hipLaunchKernelGGL(k_scatter<false>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles, adv);
+        if (scan) hipLaunchKernelGGL(k_scatter<true>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles);
+        else hipLaunchKernelGGL(k_scatter<false>, g, dim3(kBlock), 0, ctx->stream, A, ctx->n_tiles);
         CRM_TRY(t_end(ctx, CRM_KERNEL_SCATTER));
     }
-    if (!advance) {  // the gather of a step orders each voxel's arrivals itself
-        CRM_TRY(t_begin(ctx));
-        hipLaunchKernelGGL(k_fixup, dim3((Vt + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream, A);
-        CRM_TRY(t_end(ctx, CRM_KERNEL_FIXUP));
-    }
+    CRM_TRY(t_begin(ctx));
+    hipLaunchKernelGGL(k_fixup, dim3((Vt + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream, A);
+    CRM_TRY(t_end(ctx, CRM_KERNEL_FIXUP));
     CRM_TRY(t_begin(ctx));
     StateBuf src = ctx->buf[ctx->cur], dst = ctx->buf[1 - ctx->cur];
-    const uint32_t cap = ctx->cfg.solver_order;
     const bool mixed = ctx->cfg.precision == CRM_PRECISION_MIXED;
+    const StepArgs sa0 = sa ? *sa : step_args(ctx, nullptr);
     crm_status gst = CRM_OK;
     if (is_rod(ctx)) {
-        const RodArgs R = rod_args(ctx);
-        const StepArgs sa0 = sa ? *sa : step_args(ctx, nullptr);
-        const dim3 g(ctx->n_work), b(kBlock);
-        const bool ahead = keys_ahead(ctx);
-        if (ctx->D == 2) {
-            if (ahead) {
-                if (advance) hipLaunchKernelGGL((k_gather_rod<2, true, true>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-                else hipLaunchKernelGGL((k_gather_rod<2, false, true>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-            } else {
-                if (advance) hipLaunchKernelGGL((k_gather_rod<2, true, false>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-                else hipLaunchKernelGGL((k_gather_rod<2, false, false>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-            }
-        } else {
-            if (ahead) {
-                if (advance) hipLaunchKernelGGL((k_gather_rod<3, true, true>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-                else hipLaunchKernelGGL((k_gather_rod<3, false, true>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-            } else {
-                if (advance) hipLaunchKernelGGL((k_gather_rod<3, true, false>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-                else hipLaunchKernelGGL((k_gather_rod<3, false, false>), g, b, 0, ctx->stream, A, src, dst, R, sa0);
-            }
-        }
-    } else if (advance) {
-        if (ctx->D == 2)
-            gst = mixed ? launch_gather_integrate_dm<2, true>(ctx, src, dst, *sa)
-                        : launch_gather_integrate_dm<2, false>(ctx, src, dst, *sa);
-        else
-            gst = mixed ? launch_gather_integrate_dm<3, true>(ctx, src, dst, *sa)
-                        : launch_gather_integrate_dm<3, false>(ctx, src, dst, *sa);
+        if (ctx->D == 2) launch_gather_rod<2>(ctx, src, dst, false, sa0);
+        else launch_gather_rod<3>(ctx, src, dst, false, sa0);
     } else {
-        const StepArgs sa0 = sa ? *sa : step_args(ctx, nullptr);
         gst = ctx->D == 2 ? (mixed ? launch_gather_setup_d<2, true>(ctx, src, dst, sa0)
                                    : launch_gather_setup_d<2, false>(ctx, src, dst, sa0))
                           : (mixed ? launch_gather_setup_d<3, true>(ctx, src, dst, sa0)
@@ -784,10 +778,38 @@ bool keys_ahead(const crm_ctx* ctx) {
 
 crm_status launch_step(crm_ctx* ctx, const double* noise_step) {
     const StepArgs sa = step_args(ctx, noise_step);
-    const bool ahead = keys_ahead(ctx);  // the force kernel ranks the voxels
-    CRM_TRY(launch_force(ctx, ahead));
+    // the force kernel scans the next order, unless that waits for the forces or is timed
+    const bool ahead = keys_ahead(ctx), within = ahead && !timing_on(ctx);
+    CRM_TRY(launch_force(ctx, within));
     if (!ahead) CRM_TRY(launch_key(ctx, sa));
-    CRM_TRY(launch_sort(ctx, true, &sa));
+    if (!within) {
+        CRM_TRY(t_begin(ctx));
+        hipLaunchKernelGGL(k_scan_moves, dim3(ctx->n_scan), dim3(kBlock), 0, ctx->stream, arrays(ctx));
+        CRM_TRY(t_end(ctx, CRM_KERNEL_SCAN));
+    }
+    if (timing_on(ctx)) {
+        CRM_TRY(t_begin(ctx));
+        hipLaunchKernelGGL(k_next_starts, dim3((uint32_t)((ctx->Vt + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
+                           arrays(ctx));
+        CRM_TRY(t_end(ctx, CRM_KERNEL_SCATTER));
+    }
+    CRM_TRY(t_begin(ctx));
+    const StateBuf src = ctx->buf[ctx->cur], dst = ctx->buf[1 - ctx->cur];
+    const bool mixed = ctx->cfg.precision == CRM_PRECISION_MIXED;
+    crm_status st = CRM_OK;
+    if (is_rod(ctx)) {
+        if (ctx->D == 2) launch_gather_rod<2>(ctx, src, dst, true, sa);
+        else launch_gather_rod<3>(ctx, src, dst, true, sa);
+    } else if (ctx->D == 2) {
+        st = mixed ? launch_gather_integrate_dm<2, true>(ctx, src, dst, sa)
+                   : launch_gather_integrate_dm<2, false>(ctx, src, dst, sa);
+    } else {
+        st = mixed ? launch_gather_integrate_dm<3, true>(ctx, src, dst, sa)
+                   : launch_gather_integrate_dm<3, false>(ctx, src, dst, sa);
+    }
+    if (st) return st;
+    CRM_TRY(t_end(ctx, CRM_KERNEL_GATHER));
+    ctx->cur = 1 - ctx->cur;
     return CRM_OK;
 }
 
@@ -1232,7 +1254,7 @@ crm_status launch_cycle_step(crm_ctx* ctx, const double* noise_step) {
         CRM_HIP(hipGetLastError());
     }
     CRM_TRY(launch_rank(ctx));
-    CRM_TRY(launch_sort(ctx, false, &sa));
+    CRM_TRY(launch_sort(ctx, &sa, false));
     hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl);
     CRM_HIP(hipGetLastError());
     return CRM_OK;
@@ -1533,7 +1555,7 @@ crm_status remove_agents_impl(crm_ctx* ctx, const uint8_t* remove, uint64_t n_rm
     hipLaunchKernelGGL(k_remove_key, dim3((uint32_t)((n_new + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
                        arrays(ctx), ctx->buf[ctx->cur]);
     CRM_HIP(hipGetLastError());
-    CRM_TRY(launch_sort(ctx, false, nullptr));
+    CRM_TRY(launch_sort(ctx, nullptr, true));
     CRM_HIP(hipStreamSynchronize(ctx->stream));
     return check_errors(ctx, "agent removal");
 }
@@ -1611,7 +1633,7 @@ crm_status realloc_point_arrays(crm_ctx* ctx, uint64_t C) {
     }
     const uint32_t K = ctx->K;
     CRM_TRY(dalloc(ctx, ctx->d_work, C / kBlock + ctx->n_inst + 1));
-    CRM_TRY(dalloc(ctx, ctx->d_key, 2 * C));
+    CRM_TRY(dalloc(ctx, ctx->d_key, 4 * C));
     CRM_TRY(dalloc(ctx, ctx->d_rank, C));
     CRM_TRY(dalloc(ctx, ctx->d_perm, C));
     CRM_TRY(dalloc(ctx, ctx->d_force, (size_t)K * C));
@@ -1826,7 +1848,7 @@ crm_status insert_agents_impl(crm_ctx* ctx, uint64_t n, const uint64_t* mother, 
     hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)((stay_offset(ctx) + Vt + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        ctx->stream, ctx->d_count, (uint32_t)(stay_offset(ctx) + Vt), 0u);
     CRM_TRY(launch_rank(ctx));
-    CRM_TRY(launch_sort(ctx, false, nullptr));
+    CRM_TRY(launch_sort(ctx, nullptr, true));
     CRM_HIP(hipStreamSynchronize(ctx->stream));
     return check_errors(ctx, "agent insertion");
 }
@@ -2042,6 +2064,9 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
 
     const uint64_t Vt = ctx->Vt;
     ctx->n_tiles = (uint32_t)((Vt + kScanTile - 1) / kScanTile);
+    ctx->scan_shift = 0;
+    while (((uint64_t)kStepScanTiles * kScanTile << ctx->scan_shift) < Vt) ctx->scan_shift++;
+    ctx->n_scan = (uint32_t)((Vt + ((uint64_t)kScanTile << ctx->scan_shift) - 1) / ((uint64_t)kScanTile << ctx->scan_shift));
     // room for the work blocks of `C` agents (a growing cycle rebuilds the table)
     {
         const uint64_t per = is_rod(ctx) ? ctx->rods_per_block : (uint64_t)kBlock;
@@ -2049,13 +2074,13 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
         CRM_TRY(dalloc(ctx, ctx->d_work, std::max<size_t>(work.size(), Cw / per + ctx->n_inst + 1)));
     }
     CRM_TRY(dalloc(ctx, ctx->d_start, Vt + 1));
-    CRM_TRY(dalloc(ctx, ctx->d_count, stay_offset(ctx) + Vt));  // arrivals, then stayers
+    CRM_TRY(dalloc(ctx, ctx->d_count, 5 * stay_offset(ctx)));
     CRM_TRY(dalloc(ctx, ctx->d_start_local, Vt));
     CRM_TRY(dalloc(ctx, ctx->d_bsum, ctx->n_tiles + 1));
     // N-sized arrays hold `C` agents: the rods of a cycle grow up to max_agents
     const uint64_t C = (is_rod(ctx) && ctx->cycle_on) ? std::max<uint64_t>(N, ctx->cyc.max_agents) : N;
     ctx->cap_agents = C;
-    CRM_TRY(dalloc(ctx, ctx->d_key, 2 * C));
+    CRM_TRY(dalloc(ctx, ctx->d_key, 4 * C));
     CRM_TRY(dalloc(ctx, ctx->d_rank, C));
     CRM_TRY(dalloc(ctx, ctx->d_perm, C));
     CRM_TRY(dalloc(ctx, ctx->d_force, (size_t)K * C));
@@ -2096,7 +2121,7 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
     CRM_HIP(hipMemcpy(ctx->d_work, work.data(), sizeof(BlockWork) * work.size(), hipMemcpyHostToDevice));
     ctx->work_host = work;  // later rebuilds (removals) shrink it in place
     CRM_TRY(upload_tiles(ctx, tiles));
-    CRM_HIP(hipMemsetAsync(ctx->d_count, 0, sizeof(uint32_t) * (stay_offset(ctx) + Vt), ctx->stream));
+    CRM_HIP(hipMemsetAsync(ctx->d_count, 0, sizeof(uint32_t) * 5 * stay_offset(ctx), ctx->stream));
 
     // upload in agent-index order (slot = agent index before the first sort)
     ctx->cur = 0;
@@ -2160,7 +2185,7 @@ crm_status crm_set_agents(crm_ctx* ctx, const uint64_t* counts, const double* po
         hipLaunchKernelGGL(k_initial_key<3>, dim3(ctx->n_work), dim3(kBlock), 0, ctx->stream, A, S, ctx->nv);
     CRM_HIP(hipGetLastError());
     CRM_TRY(check_errors(ctx, "initial placement"));
-    CRM_TRY(launch_sort(ctx, false, nullptr));
+    CRM_TRY(launch_sort(ctx, nullptr, false));
     if (is_rod(ctx) && ctx->cycle_on)
         hipLaunchKernelGGL(k_init_vcount, dim3((uint32_t)((Vt + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
                            ctx->d_start, ctx->d_vcount, (uint32_t)Vt);

@@ -1,19 +1,22 @@
 // kernels_point.hpp -- gfx950 kernels of the per-step mechanics path for point agents.
 //
 // Step (run_sim.rs:380-403) as launched by the runtime:
-//   k_force_tiled      pair loop over the 3^D voxel stencil (update_mechanics.rs:153-238)
-//   k_key_point        next position (solvers.rs:23-347 + apply_boundary,
-//                      cartesian_cuboid_n.rs:594-631) -> next voxel index
-//                      (cartesian_cuboid_n.rs:469-491); NewtonDamped and
-//                      Langevin get it from the previous gather instead
-//   k_rank_ahead       ranks: stayers in order, arrivals atomic         } integer counting sort:
-//   k_scan_local/tiles exclusive scan of the voxel histogram, its reset } stayers keep their order,
-//   k_scatter          slot -> sorted position, final voxel starts      } movers appended by
-//   k_gather_integrate_point  arrivals put in order of previous slot,   } previous slot (sort_cells_in_voxels,
-//                      the full mechanics update written into the       }  update_mechanics.rs:418-513)
-//                      agent's new sorted slot, and the force records
-//   (set-up sorts order the arrivals with k_fixup; systems whose voxels
-//   fit one scan tile run k_sort_small, the scans and the scatter in one workgroup)
+//   k_force_tiled      pair loop over the 3^D voxel stencil (update_mechanics.rs:153-238);
+//                      further workgroups scan the next order's voxel counts (scan_moves)
+//   k_gather_integrate_point  the full mechanics update (solvers.rs:23-347 + apply_boundary,
+//                      cartesian_cuboid_n.rs:594-631) written into the agent's slot in the
+//                      next order, in which the agents that stay in a voxel keep their
+//                      order and the movers are appended by previous slot
+//                      (sort_cells_in_voxels, update_mechanics.rs:418-513); the force
+//                      records, and the voxel each agent moves to in the step after
+//                      (note_move)
+//   Brownian agents, whose next position needs the force, get that voxel from
+//   k_key_point (cartesian_cuboid_n.rs:469-491) and the scan from k_scan_moves, between the two.
+//
+// Set-up sorts (initial placement, insertion, removal, the rods' cycle) are a counting
+// sort of their own: ranks (k_initial_key, k_rank_ahead), k_scan_local/tiles, k_scatter,
+// k_fixup and k_gather_point; systems whose voxels fit one scan tile run k_sort_small, the
+// scans and the scatter in one workgroup.
 //
 // Agents live in SoA arrays sorted by voxel; a voxel's agents are the slots
 // [start[v], start[v+1]).
@@ -50,14 +53,23 @@ struct Arrays {
     const BlockWork* work;
     Control* ctrl;
     uint32_t* start;  // [Vt + 1]
-    uint32_t* start_local;  // [Vt] offset of each voxel inside its scan tile (k_scan_local)
-    uint32_t* tile_off;     // [n_tiles + 1] sum of each scan tile (k_scan_local), or its offset (k_scan_tiles)
+    uint32_t* start_local;  // [Vt] offset of each voxel inside its scan tile (k_scan_local, scan_moves)
+    uint32_t* tile_off;     // [n_tiles + 1] sum of each scan tile (k_scan_local, scan_moves), or its offset (k_scan_tiles)
+    // set-up sorts
     uint32_t* count;  // [Vt] arrivals per next voxel (atomic ranks)
-    uint32_t* stay;   // [Vt] agents binned ahead that stay in their voxel (zero otherwise)
-    uint32_t* key;    // [N] next voxel
+    uint32_t* stay;   // [Vt] agents that stay in their voxel (zero unless ranked by k_rank_ahead)
     uint32_t* rank;   // [N] arrival rank inside the next voxel
-    uint32_t* key_next;   // [N] next voxel of the following step (binned ahead by the gather)
     uint32_t* perm;   // [N] sorted slot -> previous slot
+    // the step's moves (note_move), and those of the following step that the gather notes
+    uint32_t* key;    // [N] next voxel
+    uint32_t* key_next;
+    uint32_t* head;   // [Vt] the voxel's arrivals as a list: slot + 1 of the last noted one, 0 without any
+    uint32_t* head_next;
+    uint32_t* link;   // [N] (arrivals) slot + 1 of the one noted before it
+    uint32_t* link_next;
+    int32_t* delta;   // [Vt] arrivals less departures of the voxel
+    uint32_t n_scan;      // scan tiles of the step, at most kStepScanTiles
+    uint32_t scan_shift;  // of kScanTile << scan_shift voxels
     double* force;    // [K][N]
     float* forcef;    // [K][N] in the same memory: point forces of the mixed path, stored in float
     double4* rec64;   // [N] (x, y, z, species) absolute, FP64 path
@@ -86,9 +98,8 @@ __device__ __forceinline__ void raise_error(Control* c, uint32_t kind, uint64_t 
 }
 
 // An earlier step than t raised an error.  The kernels of the steps after a
-// failing one do nothing (the ones before the sort check this, the ones after it
-// read Control::skip, set by k_scan_local), so the state stays at the end of the
-// failing step, where run_simulation! returns the error (run_sim.rs:380-403).
+// failing one do nothing, so the state stays at the end of the failing step, where
+// run_simulation! returns the error (run_sim.rs:380-403).
 __device__ __forceinline__ bool halted(const Control* c, uint64_t t) {
     return c->error_flags != 0 && (c->error_key >> 32) < t;
 }
@@ -787,6 +798,216 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t& t
     return before + inc - x;
 }
 
+// ---------------------------------------------------------------------------
+// The next order of a step.  Which voxel every agent moves to is known before the step's
+// forces (bin_ahead) or right after them (k_key_point, k_key_rod); note_move keeps, per
+// voxel, arrivals less departures and the list of arrivals.  The new voxel starts are
+// then a scan of (agents now + delta), and an agent's new slot follows from its old one:
+// a stayer's is its new voxel start plus the stayers before it in the voxel, counted with
+// wave ballots; an arrival's is counted back from the voxel's end by the arrivals' slots.
+//
+// The scan needs nothing of the forces, so it is work of further workgroups of the force
+// kernel, and the gather writes straight to the new slots: a step is two launches.  As a
+// counting sort (ranks in the force kernel, scan, scatter, gather by the sorted order) it was four,
+// each with at least 4.5 us in a chain: 50 steps of 30,000 sorting agents
+// 1.71 -> 1.33 ms, 100 of 300,000 in FP64 8.10 -> 7.36, 25 of 1600 crowded cells 1.14 ->
+// 0.93, 50 of 12,347 rods 5.50 -> 5.27.  The gather itself got slower, since its stores, not
+// its loads, are now the unaligned side (1M agents 57 -> 65 us, 4M 201 -> 227); other
+// workgroup orders and plain stores changed nothing.
+// ---------------------------------------------------------------------------
+constexpr int kScanItems = 8;
+constexpr int kScanTileLog2 = 11;
+constexpr int kScanTile = kBlock * kScanItems;
+static_assert(kScanTile == 1 << kScanTileLog2, "voxels of a scan tile");
+// Scan tiles of a step at most (two per thread of a gather workgroup, which scans their
+// sums); larger grids get tiles of 2^scan_shift times kScanTile voxels.
+constexpr uint32_t kStepScanTiles = 512;
+
+// The agent in slot s of voxel v moves to voxel k.
+__device__ __forceinline__ void note_move(int32_t* delta, uint32_t* head, uint32_t* link, uint32_t s, uint32_t v,
+                                          uint32_t k) {
+    if (k == v) return;
+    atomicAdd(&delta[v], -1);
+    atomicAdd(&delta[k], 1);
+    link[s] = atomicExch(&head[k], s + 1u);
+}
+
+// Offsets of the tile's voxels inside it (start_local) and its sum (tile_off) in the
+// next order; clears delta for the next step's moves, and the lists that they go to.
+__device__ __forceinline__ void scan_moves(const Arrays& A, uint32_t tile) {
+    static_assert(kScanItems == 8, "two 16-byte accesses per group");
+    const uint32_t Vt = A.Vt;
+    uint32_t carry = 0;
+    for (uint32_t c = 0; c < (1u << A.scan_shift); c++) {
+        const uint64_t base = (((uint64_t)tile << A.scan_shift) + c) * kScanTile + (uint64_t)threadIdx.x * kScanItems;
+        uint32_t vals[kScanItems], sum = 0;
+        const bool whole = base + kScanItems <= Vt;
+        if (whole) {  // (start, delta, head and start_local are 256-byte aligned)
+            const uint4* b4 = reinterpret_cast<const uint4*>(A.start + base);
+            int4* d4 = reinterpret_cast<int4*>(A.delta + base);
+            uint4* h4 = reinterpret_cast<uint4*>(A.head_next + base);
+            const uint4 b0 = b4[0], b1 = b4[1];
+            const uint32_t e = A.start[base + kScanItems];
+            const int4 d0 = d4[0], d1 = d4[1];
+            vals[0] = b0.y - b0.x + (uint32_t)d0.x;
+            vals[1] = b0.z - b0.y + (uint32_t)d0.y;
+            vals[2] = b0.w - b0.z + (uint32_t)d0.z;
+            vals[3] = b1.x - b0.w + (uint32_t)d0.w;
+            vals[4] = b1.y - b1.x + (uint32_t)d1.x;
+            vals[5] = b1.z - b1.y + (uint32_t)d1.y;
+            vals[6] = b1.w - b1.z + (uint32_t)d1.z;
+            vals[7] = e - b1.w + (uint32_t)d1.w;
+            d4[0] = d4[1] = make_int4(0, 0, 0, 0);
+            h4[0] = h4[1] = make_uint4(0u, 0u, 0u, 0u);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kScanItems; i++) {
+                const uint64_t q = base + i;
+                vals[i] = q < Vt ? A.start[q + 1] - A.start[q] + (uint32_t)A.delta[q] : 0u;
+                if (q < Vt) {
+                    A.delta[q] = 0;
+                    A.head_next[q] = 0u;
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) sum += vals[i];
+        uint32_t total;
+        uint32_t run = carry + block_exclusive_scan(sum, total);
+        carry += total;
+        uint32_t out[kScanItems];
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) {
+            out[i] = run;
+            run += vals[i];
+        }
+        if (whole) {
+            uint4* o4 = reinterpret_cast<uint4*>(A.start_local + base);
+            o4[0] = make_uint4(out[0], out[1], out[2], out[3]);
+            o4[1] = make_uint4(out[4], out[5], out[6], out[7]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kScanItems; i++)
+                if (base + i < Vt) A.start_local[base + i] = out[i];
+        }
+    }
+    if (threadIdx.x == 0) {
+        A.tile_off[tile] = carry;
+        if (tile == 0) A.ctrl->gather_step = A.ctrl->step;
+    }
+}
+
+// In place of the scan after an error: the gather finds the step that is not to run (with
+// the failing step's number in gather_step it would run again).
+__device__ __forceinline__ void skip_scan(const Arrays& A) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) A.ctrl->gather_step = A.ctrl->step;
+}
+
+__global__ __launch_bounds__(kBlock) void k_scan_moves(Arrays A) {
+    if (halted(A.ctrl, A.ctrl->step)) skip_scan(A);
+    else scan_moves(A, blockIdx.x);
+}
+
+// An agent's old voxel v, its next voxel k, and the stayers of v in the slots before its own.
+struct Move {
+    uint32_t v, k, r;
+};
+
+// The moves of slots first + threadIdx.x for threadIdx.x < count; called by whole
+// workgroups.  Slots are sorted by voxel, so a voxel's slots in a wave are one run of
+// lanes; the part of the first lane's voxel before the wave is looked up by all lanes.
+__device__ __forceinline__ Move move_of(const Arrays& A, const uint32_t* __restrict__ vox, uint32_t first,
+                                        uint32_t count) {
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x & ~63u, w0 = first + w;
+    const bool live = threadIdx.x < count;
+    Move m{0xffffffffu, 0xffffffffu, 0u};
+    if (live) {
+        m.v = vox[first + threadIdx.x];
+        m.k = A.key[first + threadIdx.x];
+    }
+    uint32_t base = w0;
+    bool ok = w < count && base > lane;
+    uint32_t vb = ok ? vox[base - 1u - lane] : 0u, kb = ok ? A.key[base - 1u - lane] : 0u;
+    const uint32_t v0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.v);
+    ok = ok && vb == v0;
+    uint32_t before = (uint32_t)__popcll(__ballot(ok && kb == v0));
+    while (__ballot(ok) == ~0ull) {  // more than 64 of them
+        base -= 64u;
+        ok = base > lane;
+        vb = ok ? vox[base - 1u - lane] : 0u;
+        kb = ok ? A.key[base - 1u - lane] : 0u;
+        ok = ok && vb == v0;
+        before += (uint32_t)__popcll(__ballot(ok && kb == v0));
+    }
+    const uint32_t vp = __shfl_up(m.v, 1, 64);
+    const uint64_t runs = __ballot(lane == 0u || m.v != vp), stay = __ballot(live && m.k == m.v);
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t h = 63u - (uint32_t)__clzll((long long)(runs & (below | (1ull << lane))));  // the run's first lane
+    m.r = (uint32_t)__popcll(stay & below & ~((1ull << h) - 1ull)) + (h == 0u ? before : 0u);
+    return m;
+}
+
+// Offsets of the scan tiles, from their sums, in s_off[kStepScanTiles].
+__device__ __forceinline__ void step_tile_offsets(const Arrays& A, uint32_t* s_off) {
+    if (A.n_scan == 1u) {
+        if (threadIdx.x == 0) s_off[0] = 0u;
+    } else {
+        const uint32_t q = 2u * threadIdx.x;
+        const uint32_t x = q < A.n_scan ? A.tile_off[q] : 0u, y = q + 1u < A.n_scan ? A.tile_off[q + 1u] : 0u;
+        uint32_t total;
+        const uint32_t ex = block_exclusive_scan(x + y, total);
+        s_off[q] = ex;
+        s_off[q + 1u] = ex + x;
+    }
+    __syncthreads();
+}
+
+// Voxel v's start in the next order (sl = start_local[v]).
+__device__ __forceinline__ uint32_t next_start(const Arrays& A, const uint32_t* s_off, uint32_t v, uint32_t sl) {
+    return sl + s_off[v >> (kScanTileLog2 + A.scan_shift)];
+}
+
+// Slot in the next order of the agent in slot g with move m (sl = start_local[m.k]).
+__device__ __forceinline__ uint32_t next_slot(const Arrays& A, const uint32_t* s_off, uint32_t g, const Move& m,
+                                              uint32_t sl) {
+    if (m.k == m.v) return next_start(A, s_off, m.k, sl) + m.r;
+    uint32_t n = 0, before = 0;
+    for (uint32_t j = A.head[m.k]; j != 0u; j = A.link[j - 1u]) {
+        n++;
+        before += j - 1u < g ? 1u : 0u;
+    }
+    const uint32_t e = m.k + 1u < A.Vt ? next_start(A, s_off, m.k + 1u, A.start_local[m.k + 1u]) : (uint32_t)A.N;
+    return e - n + before;
+}
+
+// The workgroup's share of the new voxel starts (sl = start_local of its thread's first).
+__device__ __forceinline__ void write_starts(const Arrays& A, const uint32_t* s_off, uint32_t sl) {
+    const uint64_t v0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x, step = (uint64_t)gridDim.x * kBlock;
+    if (v0 < A.Vt) A.start[v0] = next_start(A, s_off, (uint32_t)v0, sl);
+    for (uint64_t v = v0 + step; v < A.Vt; v += step) A.start[v] = next_start(A, s_off, (uint32_t)v, A.start_local[v]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) A.start[A.Vt] = (uint32_t)A.N;
+}
+__device__ __forceinline__ uint32_t first_start_local(const Arrays& A) {
+    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    return v < A.Vt ? A.start_local[v] : 0u;
+}
+
+// The gather's last duty towards the order: the new starts and the completed step (the
+// gather itself reads gather_step).
+__device__ __forceinline__ void finish_order(const Arrays& A, const uint32_t* s_off, uint32_t sl, uint64_t t) {
+    write_starts(A, s_off, sl);
+    if (blockIdx.x == 0 && threadIdx.x == 0) A.ctrl->step = t + 1;
+}
+
+// The new starts on their own, ahead of the gather that writes them again: in contexts
+// that time the kernel classes, whose scan is a launch of its own as well.
+__global__ __launch_bounds__(kBlock) void k_next_starts(Arrays A) {
+    __shared__ uint32_t s_off[kStepScanTiles];
+    if (halted(A.ctrl, A.ctrl->gather_step)) return;
+    step_tile_offsets(A, s_off);
+    write_starts(A, s_off, first_start_local(A));
+}
+
 // a / d for a < 2^14, 0 < d <= 64, with d's float reciprocal: (a + 1/2) / d keeps a
 // fractional part >= 1/128 that the two float roundings cannot carry across.
 __device__ __forceinline__ uint32_t small_div(uint32_t a, float inv_d) {
@@ -804,14 +1025,21 @@ template <int D, int POT, bool MIXED, bool SENSE, bool MULTI>
 __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A, StateBuf S,
                                                                      const ForceTile* __restrict__ tiles,
                                                                      uint32_t physical, uint32_t symmetric,
-                                                                     uint32_t no_lds, uint32_t rank,
+                                                                     uint32_t no_lds, uint32_t n_scan,
                                                                      uint32_t lanes_log2) {
     const uint32_t lg = MULTI ? lanes_log2 : 0u;
     using Rec = typename RecOf<MIXED>::type;
     using Recs = LdsRecords<D, MIXED>;
     constexpr int CAP = Recs::kCap;
     constexpr uint32_t NP = D == 3 ? 3u : 1u;         // staged planes
-    const ForceTile T = tiles[xcd_block(blockIdx.x, gridDim.x)];  // loaded beside the control block
+    // the first n_scan workgroups scan the voxel counts (behind the others: 1M sorting agents
+    // 77.8 -> 79.8 us; by the first tiles' workgroups themselves: 4M-agent lattice 495 -> 519)
+    if (blockIdx.x < n_scan) {
+        if (halted(A.ctrl, A.ctrl->step)) skip_scan(A);
+        else scan_moves(A, blockIdx.x);
+        return;
+    }
+    const ForceTile T = tiles[xcd_block(blockIdx.x - n_scan, gridDim.x - n_scan)];  // loaded beside the control block
     if (halted(A.ctrl, A.ctrl->step)) return;
     constexpr uint32_t PA_OWN = D == 3 ? 1u : 0u;     // the tile's own plane among them
     __shared__ __align__(16) char lds[Recs::kTotal];
@@ -846,31 +1074,6 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
     const uint32_t n_vox = G.RW * G.NC * NP;
     const uint32_t n_ownv = R * W;
     const bool fits = !no_lds && n_vox < (uint32_t)kLdsVoxelStarts && n_ownv <= (uint32_t)kOwnVoxMax;
-
-    // The step's re-binning ranks for the tile's own voxels (k_rank_ahead's work;
-    // the tiles cover every voxel once): an agent whose next voxel, binned ahead by
-    // the previous gather, is its current one takes the next stayer rank in slot
-    // order, the others an atomic arrival rank in their next voxel.  The force
-    // computation reads none of key, rank, stay or count, so each wave does this
-    // after its agents' forces, beside the waves still computing theirs.
-    // staged: the own voxels' slot ranges are in LDS (own_gs, own_pre) already.
-    auto rank_tile = [&](bool staged) {
-        if (!rank) return;
-        const float inv_w = 1.0f / (float)W;
-        for (uint32_t u = threadIdx.x; u < n_ownv; u += kBlock) {
-            const uint32_t r = small_div(u, inv_w), c = u - r * W;
-            const uint32_t g = voff + (T.a0 * n1 + T.b0 + r) * n2 + T.c0 + c;
-            const uint32_t b = staged ? own_gs[u] : A.start[g];
-            const uint32_t e = staged ? b + ((uint32_t)own_pre[u + 1] - (uint32_t)own_pre[u]) : A.start[g + 1];
-            uint32_t n = 0;
-            for (uint32_t s = b; s < e; s++) {
-                const uint32_t k = A.key[s];
-                if (k == g) A.rank[s] = n++;
-                else A.rank[s] = kMoved | atomicAdd(&A.count[k], 1u);
-            }
-            A.stay[g] = n;
-        }
-    };
 
     if (fits) {
         // staged voxel v = (rb * NC + c - cl) * NP + pa; thread t holds v = 3t .. 3t + 2
@@ -1103,7 +1306,6 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                                                       physical, symmetric, src, unit, MULTI ? threadIdx.x & gmask : 0u,
                                                       lg);
                 }
-                rank_tile(true);
                 return;
             }
             for (uint32_t t = threadIdx.x; t < (n_own << lg); t += kBlock) {
@@ -1114,7 +1316,6 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
                 agent_force<D, POT, MIXED, SENSE>(A, S, P, s, self, src.record(self, w), ov, w, physical, symmetric, src, unit,
                                                   MULTI ? t & gmask : 0u, lg);
             }
-            rank_tile(true);
             return;
         }
     }
@@ -1147,7 +1348,6 @@ __global__ __launch_bounds__(kBlock, MIXED ? 5 : 4) void k_force_tiled(Arrays A,
             agent_force<D, POT, MIXED, SENSE>(A, S, P, s, s, src.record(s, wm), ov, w, physical, symmetric, src, unit);
         }
     }
-    rank_tile(false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1341,7 +1541,7 @@ __device__ __forceinline__ bool point_step(const InstParams& P, const StepArgs& 
 }
 
 // Next voxel of every agent (get_index_of, cartesian_cuboid_n.rs:469-491) from
-// the position it will have after this step (k_rank_ahead ranks it).  A
+// the position it will have after this step.  A
 // position whose index has no voxel keeps the old one (update_mechanics.rs:430-453).
 template <int D, int MECH>
 __global__ __launch_bounds__(kBlock) void k_key_point(Arrays A, StateBuf S, StepArgs sa) {
@@ -1378,7 +1578,8 @@ __global__ __launch_bounds__(kBlock) void k_key_point(Arrays A, StateBuf S, Step
         key = S.vox[s];
         atomicAdd((unsigned long long*)&A.ctrl->out_of_grid, 1ull);
     }
-    A.key[s] = key;  // ranked by k_rank_ahead
+    A.key[s] = key;
+    note_move(A.delta, A.head, A.link, (uint32_t)s, S.vox[s], key);
 }
 
 // Initial binning (Domain::decompose, concepts-derive/src/domain.rs:357-380 with
@@ -1423,12 +1624,8 @@ __global__ __launch_bounds__(kBlock) void k_initial_key(Arrays A, StateBuf S, ui
 }
 
 // ---------------------------------------------------------------------------
-// Counting sort by voxel.
+// Counting sort by voxel (set-up sorts).
 // ---------------------------------------------------------------------------
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kBlock * kScanItems;
-
-
 // Each thread scans kScanItems consecutive voxels of count + stay into their
 // offsets inside the scan tile (start_local) and clears count for the next step's
 // ranks; whole groups move as two 16-byte loads per array and two 16-byte stores
@@ -1511,17 +1708,15 @@ __global__ __launch_bounds__(kBlock) void k_scan_tiles(uint32_t* __restrict__ bs
 // Thread g writes the final start of voxel g (tile-local offset + tile offset) and
 // places agent g in the slot list of its next voxel: a stayer at its rank, an
 // arrival (kMoved) after the voxel's stayers in atomic order.  Launched over
-// max(N, Vt) threads.  Thread 0 writes start[Vt]; advance != 0 also completes the
-// step counter (every kernel that reads it for this step has run; the gather reads
-// the new value).
+// max(N, Vt) threads.  Thread 0 writes start[Vt].
 // SCAN: every workgroup scans the tile sums itself (two per thread): one more dependent
 // load and two barriers in place of k_scan_tiles, a 4.5 us launch in a chain of small
-// kernels.  The scatter stays at 4.7 us for 30,000 and 4.9 for 300,000 agents (a
-// 30,000-agent step 32.5 -> 28.9 us) and goes from 6.0 to 7.5 for 1M in 432 tiles; with
-// 1728 tiles per workgroup the step lost 1.7 %, hence the line at two per thread.
+// kernels.  The scatter stays at 4.7 us for 30,000 and 4.9 for 300,000 agents and goes
+// from 6.0 to 7.5 for 1M in 432 tiles; with 1728 tiles per workgroup it lost more than
+// the launch, hence the line at two per thread.
 constexpr uint32_t kScatterTiles = 512;
 template <bool SCAN>
-__global__ __launch_bounds__(kBlock) void k_scatter(Arrays A, uint32_t n_tiles, uint32_t advance) {
+__global__ __launch_bounds__(kBlock) void k_scatter(Arrays A, uint32_t n_tiles) {
     if (A.ctrl->skip) return;
     __shared__ uint32_t s_off[SCAN ? kScatterTiles : 1];
     uint32_t total = 0;
@@ -1536,10 +1731,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter(Arrays A, uint32_t n_tiles, 
         off = s_off;
     }
     const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (g == 0) {
-        A.start[A.Vt] = SCAN ? total : A.tile_off[n_tiles];
-        if (advance) A.ctrl->step += 1;
-    }
+    if (g == 0) A.start[A.Vt] = SCAN ? total : A.tile_off[n_tiles];
     if (g < A.Vt) A.start[g] = A.start_local[g] + off[g / kScanTile];
     if (g >= A.N) return;
     const uint32_t k = A.key[g], r = A.rank[g];
@@ -1550,9 +1742,9 @@ __global__ __launch_bounds__(kBlock) void k_scatter(Arrays A, uint32_t n_tiles, 
 // Small systems (every voxel in one scan tile, at most kSmallSortAgents agents):
 // k_scan_local, k_scan_tiles and k_scatter in one workgroup, with barriers in place
 // of the launches between them; the voxel starts stay in LDS for the scatter.  The
-// same skip flag, count reset, starts, start[Vt], step advance and slot lists.
+// same skip flag, count reset, starts, start[Vt] and slot lists.
 constexpr uint32_t kSmallSortAgents = 16384;
-__global__ __launch_bounds__(kBlock) void k_sort_small(Arrays A, uint32_t advance) {
+__global__ __launch_bounds__(kBlock) void k_sort_small(Arrays A) {
     static_assert(kScanItems == 8, "eight voxels per thread");
     __shared__ uint32_t s_start[kScanTile];
     const bool skip = halted(A.ctrl, A.ctrl->step);
@@ -1579,10 +1771,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_small(Arrays A, uint32_t advanc
         }
         run += vals[i];
     }
-    if (threadIdx.x == 0) {
-        A.start[Vt] = total;
-        if (advance) A.ctrl->step += 1;
-    }
+    if (threadIdx.x == 0) A.start[Vt] = total;
     __syncthreads();
     for (uint32_t g = threadIdx.x; g < (uint32_t)A.N; g += kBlock) {
         const uint32_t k = A.key[g], r = A.rank[g];
@@ -1596,8 +1785,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_small(Arrays A, uint32_t advanc
 // their order and the movers are appended in order of old voxel, then old position
 // (sort_cells_in_voxels_step_1/2, update_mechanics.rs:418-513).  Set-up sorts rank
 // every agent atomically with stay = 0 and get the whole voxel in order of previous
-// slot.  The point gather of a step orders the arrivals itself (arrival_slot), so
-// the step's sort launches this kernel only for rods.
+// slot.
 __global__ __launch_bounds__(kBlock) void k_fixup(Arrays A) {
     if (A.ctrl->skip) return;
     const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -1616,18 +1804,6 @@ __global__ __launch_bounds__(kBlock) void k_fixup(Arrays A) {
         }
         A.perm[j] = x;
     }
-}
-
-// Slot of the agent from previous slot o that k_scatter put at slot i of voxel key:
-// an arrival (kMoved rank) belongs after the voxel's stayers at the number of the
-// voxel's arrivals with a smaller previous slot, the order k_fixup gives.
-__device__ __forceinline__ uint32_t arrival_slot(const Arrays& A, uint32_t i, uint32_t o, uint32_t key) {
-    if (!(A.rank[o] & kMoved)) return i;
-    const uint32_t m = A.start[key] + A.stay[key], e = A.start[key + 1];
-    if (e - m < 2u) return i;
-    uint32_t r = 0;
-    for (uint32_t j = m; j < e; j++) r += A.perm[j] < o ? 1u : 0u;
-    return m + r;
 }
 
 // Force record of slot s: absolute double coordinates (FP64), or 30-bit fixed
@@ -1688,16 +1864,19 @@ __device__ __forceinline__ void bin_ahead(const Arrays& A, const InstParams& P, 
     if (ok) key = P.voxel_offset + (idx[0] * P.n[1] + idx[1]) * P.n[2] + idx[2];
     else atomicAdd((unsigned long long*)&A.ctrl->out_of_grid, 1ull);
     A.key_next[s] = key;
+    note_move(A.delta, A.head_next, A.link_next, (uint32_t)s, vox, key);
 }
 
-// Ranks of the next voxels (binned ahead by the gather, or by a key kernel after
-// the forces), with an atomic only for agents that change voxel.  Thread per
-// voxel v of the current order: the agents of v that stay get consecutive ranks
-// in slot order and their number goes to stay[v]; the others take an atomic rank
-// among the arrivals of their next voxel (count), flagged with kMoved, which the
-// scatter places after that voxel's stayers; k_fixup (set-up sorts) or the gather
-// puts the arrivals in order.
-__device__ __forceinline__ void rank_voxel(const Arrays& A, uint32_t v) {
+// Ranks of a set-up sort whose agents are in voxel order already (insertion, the rods'
+// cycle), with an atomic only for agents that change voxel.  Thread per voxel v of the
+// current order: the agents of v that stay get consecutive ranks in slot order and
+// their number goes to stay[v]; the others take an atomic rank among the arrivals of
+// their next voxel (count), flagged with kMoved, which the scatter places after that
+// voxel's stayers; k_fixup puts the arrivals in order.
+__global__ __launch_bounds__(kBlock) void k_rank_ahead(Arrays A) {
+    if (halted(A.ctrl, A.ctrl->step)) return;
+    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (v >= A.Vt) return;
     const uint32_t b = A.start[v], e = A.start[v + 1];
     uint32_t n = 0;
     for (uint32_t s = b; s < e; s++) {
@@ -1706,12 +1885,6 @@ __device__ __forceinline__ void rank_voxel(const Arrays& A, uint32_t v) {
         else A.rank[s] = kMoved | atomicAdd(&A.count[k], 1u);
     }
     A.stay[v] = n;
-}
-
-__global__ __launch_bounds__(kBlock) void k_rank_ahead(Arrays A) {
-    if (halted(A.ctrl, A.ctrl->step)) return;
-    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (v < A.Vt) rank_voxel(A, (uint32_t)v);
 }
 
 // Permutes the state into sorted order and writes the force records, without
@@ -1760,25 +1933,25 @@ __global__ __launch_bounds__(kBlock) void k_gather_point(Arrays A, StateBuf src,
     if constexpr (AHEAD) bin_ahead<D, MECH>(A, P, sa, t, id, s, p, v, r0, r1, key, birth);
 }
 
-// Gather + integrate: thread i moves the agent from slot o = perm[i] to its sorted
-// slot s (i itself, or arrival_slot's place among the voxel's arrivals); its
-// update (the same point_step as in k_key_point, so the same position) is computed
-// here and the new state written straight to slot s, together with the force
-// record for the next step.  The scatter has already advanced the step counter,
-// so this step started after step - 1 steps.
+// Gather + integrate: the thread of slot o computes its agent's update (the same
+// point_step as in k_key_point, so the same position) and writes the new state to the
+// agent's slot s in the next order, together with the force record for the next step.
+// It runs at the memory's rate: the state is read in slot order, so the loads wait for
+// no other load, and the slots written are those read, shifted by the few arrivals.
 template <int D, bool MIXED, int MECH>
 __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, StateBuf src, StateBuf dst,
                                                                      StepArgs sa) {
-    if (A.ctrl->skip) return;
+    __shared__ uint32_t s_off[kStepScanTiles];
+    const uint64_t t = A.ctrl->gather_step;
     const BlockWork w = A.work[blockIdx.x];
-    if (threadIdx.x >= w.count) return;
-    const uint32_t i = (uint32_t)(w.first + threadIdx.x);
+    if (halted(A.ctrl, t)) return;
     const InstParams& P = A.ip[w.inst];
     const uint64_t N = A.N;
-    const uint64_t t = A.ctrl->step - 1;
-    const uint32_t o = A.perm[i];
-    const uint32_t key = A.key[o];
-    const uint64_t s = arrival_slot(A, i, o, key);
+    const Move m = move_of(A, src.vox, (uint32_t)w.first, w.count);
+    const uint32_t key = m.k;
+    const bool in_block = threadIdx.x < w.count;
+    const uint32_t o = (uint32_t)w.first + min(threadIdx.x, w.count - 1u);
+    const uint32_t sl = in_block ? A.start_local[key] : 0u, sl0 = first_start_local(A);
     const uint32_t id = src.id[o];
     const uint64_t birth = src.birth ? src.birth[o] : 0u;
     const Ring rg = ring_agent(t, birth, sa.cap, sa.newest_first);
@@ -1805,48 +1978,53 @@ __global__ __launch_bounds__(kBlock) void k_gather_integrate_point(Arrays A, Sta
             hv[h][k] = live ? __builtin_nontemporal_load(&src.hdv[e]) : 0.0;
         }
     }
-    auto hist = [&](int i, int k, bool is_dv) {
-        const uint32_t sl = rg.it[i];
-        return is_dv ? (sl ? hv[1][k] : hv[0][k]) : (sl ? hx[1][k] : hx[0][k]);
-    };
-    const bool out = point_step<D, MECH, true>(P, sa, rg, t, id, x, v, f, hist, nx, nv, dx, dv);
-    if (out) raise_error(A.ctrl, CRM_BOUNDARY_ERROR, t, id);
+    step_tile_offsets(A, s_off);
+    if (in_block) {
+        const uint64_t s = next_slot(A, s_off, o, m, sl);
+        auto hist = [&](int i, int k, bool is_dv) {
+            const bool second = rg.it[i] != 0u;
+            return is_dv ? (second ? hv[1][k] : hv[0][k]) : (second ? hx[1][k] : hx[0][k]);
+        };
+        const bool out = point_step<D, MECH, true>(P, sa, rg, t, id, x, v, f, hist, nx, nv, dx, dv);
+        if (out) raise_error(A.ctrl, CRM_BOUNDARY_ERROR, t, id);
 #pragma unroll
-    for (int k = 0; k < D; k++) {
-        __builtin_nontemporal_store(nx[k], &dst.pos[k * N + s]);
-        __builtin_nontemporal_store(nv[k], &dst.vel[k * N + s]);
-    }
-    // ring: the slot written this step gets (dx, dv).  The other slot's entry, which
-    // the next step overwrites before it reads the ring, is carried over by the last
-    // step of a call only (48 of 332 bytes per 3-D agent; a call that ends early at
-    // an error gets it from k_carry_ring)
-    if (rg.cap > 0) {
-        const bool both = n_old > 0 && t >= A.ctrl->last_step;
+        for (int k = 0; k < D; k++) {
+            __builtin_nontemporal_store(nx[k], &dst.pos[k * N + s]);
+            __builtin_nontemporal_store(nv[k], &dst.vel[k * N + s]);
+        }
+        // ring: the slot written this step gets (dx, dv).  The other slot's entry, which
+        // the next step overwrites before it reads the ring, is carried over by the last
+        // step of a call only (48 of 332 bytes per 3-D agent; a call that ends early at
+        // an error gets it from k_carry_ring)
+        if (rg.cap > 0) {
+            const bool both = n_old > 0 && t >= A.ctrl->last_step;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const bool keep = (uint32_t)h < rg.cap && ((uint32_t)h == rg.wslot || both);
+            for (int h = 0; h < 2; h++) {
+                const bool keep = (uint32_t)h < rg.cap && ((uint32_t)h == rg.wslot || both);
 #pragma unroll
-            for (int k = 0; k < D; k++) {
-                if (h == (int)rg.wslot) {
-                    hx[h][k] = dx[k];
-                    hv[h][k] = dv[k];
-                }
-                if (keep) {
-                    const uint64_t e = ((uint64_t)h * D + k) * N + s;
-                    __builtin_nontemporal_store(hx[h][k], &dst.hdx[e]);
-                    __builtin_nontemporal_store(hv[h][k], &dst.hdv[e]);
+                for (int k = 0; k < D; k++) {
+                    if (h == (int)rg.wslot) {
+                        hx[h][k] = dx[k];
+                        hv[h][k] = dv[k];
+                    }
+                    if (keep) {
+                        const uint64_t e = ((uint64_t)h * D + k) * N + s;
+                        __builtin_nontemporal_store(hx[h][k], &dst.hdx[e]);
+                        __builtin_nontemporal_store(hv[h][k], &dst.hdv[e]);
+                    }
                 }
             }
         }
+        const int32_t sp = src.species[o];
+        dst.species[s] = sp;
+        dst.id[s] = id;
+        dst.vox[s] = key;
+        write_record<D, MIXED>(A, P, s, key, nx, sp);
+        if (dst.birth) dst.birth[s] = (uint32_t)birth;
+        if constexpr (MECH != CRM_MECHANICS_BROWNIAN)
+            bin_ahead<D, MECH>(A, P, sa, t + 1, id, s, nx, nv, hx[0], hx[1], key, birth);
     }
-    const int32_t sp = src.species[o];
-    dst.species[s] = sp;
-    dst.id[s] = id;
-    dst.vox[s] = key;
-    write_record<D, MIXED>(A, P, s, key, nx, sp);
-    if (dst.birth) dst.birth[s] = (uint32_t)birth;
-    if constexpr (MECH != CRM_MECHANICS_BROWNIAN)
-        bin_ahead<D, MECH>(A, P, sa, t + 1, id, s, nx, nv, hx[0], hx[1], key, birth);
+    finish_order(A, s_off, sl0, t);
 }
 
 // Agents that were put in a voxel their position is not in (inserted ones).
@@ -1856,13 +2034,16 @@ __global__ void k_note_out_of_grid(Control* c, uint64_t n) { c->out_of_grid += n
 __global__ void k_set_last_step(Control* c, uint64_t t) { c->last_step = t; }
 
 // After a call that ended at an error before its last step t: the older ring entry of
-// every agent, from the failing step's source buffer (the sort's arrays still hold that
-// step's order) to its destination.  K components per agent.
+// every agent, from the failing step's source buffer (the moves and the scan still hold
+// that step's) to its destination.  K components per agent.
 __global__ __launch_bounds__(kBlock) void k_carry_ring(Arrays A, StateBuf src, StateBuf dst, uint64_t t, uint32_t K) {
-    const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= A.N) return;
-    const uint32_t o = A.perm[i];
-    const uint64_t s = arrival_slot(A, (uint32_t)i, o, A.key[o]);
+    __shared__ uint32_t s_off[kStepScanTiles];
+    const uint32_t first = blockIdx.x * kBlock, count = (uint32_t)min<uint64_t>(kBlock, A.N - first);
+    const Move m = move_of(A, src.vox, first, count);
+    step_tile_offsets(A, s_off);
+    if (threadIdx.x >= count) return;
+    const uint32_t o = first + threadIdx.x;
+    const uint64_t s = next_slot(A, s_off, o, m, A.start_local[m.k]);
     if (t <= (src.birth ? src.birth[o] : 0u)) return;  // no older entry
     const uint64_t h = 1u - (t & 1u);
     for (uint32_t k = 0; k < K; k++) {

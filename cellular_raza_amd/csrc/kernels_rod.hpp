@@ -68,8 +68,11 @@ __device__ __forceinline__ bool rod_lane(const BlockWork& w, uint32_t nv, uint64
 constexpr uint32_t kRodLdsBytes = 36 * 1024;
 template <int D, int POT, bool MIXED>
 __global__ __launch_bounds__(kBlock, 4) void k_force_rod(Arrays A, StateBuf S, RodArgs R, uint32_t physical,
-                                                          uint32_t no_lds, uint32_t rank) {
-    if (halted(A.ctrl, A.ctrl->step)) return;
+                                                          uint32_t no_lds, uint32_t n_scan) {
+    if (halted(A.ctrl, A.ctrl->step)) {
+        skip_scan(A);
+        return;
+    }
     const BlockWork w = A.work[blockIdx.x];
     uint64_t s;
     uint32_t v;
@@ -562,13 +565,10 @@ __global__ __launch_bounds__(kBlock, 4) void k_force_rod(Arrays A, StateBuf S, R
         if (staged) work(std::true_type{});
         else work(std::false_type{});
     }
-    // the step's re-binning ranks (k_rank_ahead's work: keys binned ahead, which the
-    // forces do not read), a share of the voxels per workgroup; each wave comes here
-    // after its own forces (ahead of them the ranks' loads delayed every workgroup:
-    // 200,000 rods 326 -> 357 us)
-    if (rank)
-        for (uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x; g < A.Vt; g += (uint64_t)gridDim.x * kBlock)
-            rank_voxel(A, (uint32_t)g);
+    // the scan of the next order, a tile for each of the first workgroups after its forces
+    // (workgroups of its own behind the others: 200,000 rods 333 -> 358 us; ahead of them:
+    // 12,347 rods 85 -> 91)
+    for (uint32_t q = blockIdx.x; q < n_scan; q += gridDim.x) scan_moves(A, q);
 }
 
 // Normal k of a rod's K normals for (agent, step): Philox block k / 2, element k % 2.
@@ -824,7 +824,8 @@ __global__ __launch_bounds__(kBlock) void k_key_rod(Arrays A, StateBuf S, RodArg
         key = S.vox[s];
         atomicAdd((unsigned long long*)&A.ctrl->out_of_grid, 1ull);
     }
-    A.key[s] = key;  // ranked by k_rank_ahead
+    A.key[s] = key;
+    note_move(A.delta, A.head, A.link, (uint32_t)s, S.vox[s], key);
 }
 
 // Per-rod fields that follow the rod through a sort or a re-layout (strides of
@@ -861,8 +862,8 @@ __device__ __forceinline__ void rod_ahead(const InstParams& P, const StepArgs& s
     for (int k = 0; k < D; k++) out[k] = nx[k];
 }
 
-// Gather + integrate for rods: lane (s, v) computes vertex row v of the rod that
-// lands in sorted slot s (coming from slot o).  With AHEAD it also bins
+// Gather + integrate for rods: lane (o, v) computes vertex row v of the rod in slot o,
+// which goes to slot s of the next order (set-up: from slot o = perm[s]).  With AHEAD it also bins
 // the rod for the next step, as k_key_rod would after that step's forces: the
 // position update needs neither the force nor noise other than the next step's
 // (Philox, or none), so the new vertex positions, velocities and ring give the
@@ -873,7 +874,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
     __shared__ double newpos[kRodLdsK];
     __shared__ double win[INTEGRATE ? kRodWinK : 1];
     __shared__ double aheadpos[AHEAD ? kRodLdsK : 1];
-    if (A.ctrl->skip) return;
+    __shared__ uint32_t s_off[INTEGRATE ? kStepScanTiles : 1];
+    const uint64_t t = INTEGRATE ? A.ctrl->gather_step : 0u;
+    if (INTEGRATE ? halted(A.ctrl, t) : A.ctrl->skip != 0u) return;
     const BlockWork w = A.work[blockIdx.x];
     const uint32_t nv = R.nv, K = nv * D;
     // rods fastest across the lanes: thread t takes vertex row t / rpb of the
@@ -882,13 +885,21 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
     // streams read or written once (forces, the new state and ring) bypass the
     // caches' retention (nontemporal; 200,000 2-D rods 125 -> 118 us); positions stay cached, the
     // neighbouring vertex rows read them again.
-    // The rods of a step come in the order of k_scatter: an arrival's sorted slot is
-    // arrival_slot's (looked up once per rod).
     __shared__ uint32_t s_src[kBlock], s_dst[kBlock];
-    if (threadIdx.x < w.count) {
-        const uint32_t i = (uint32_t)w.first + threadIdx.x, o = A.perm[i];
-        s_src[threadIdx.x] = o;
-        s_dst[threadIdx.x] = INTEGRATE ? arrival_slot(A, i, o, A.key[o]) : i;
+    uint32_t sl0 = 0;
+    if constexpr (INTEGRATE) {
+        const Move m = move_of(A, src.vox, (uint32_t)w.first, w.count);
+        sl0 = first_start_local(A);
+        step_tile_offsets(A, s_off);
+        if (threadIdx.x < w.count) {
+            const uint32_t o = (uint32_t)w.first + threadIdx.x;
+            s_src[threadIdx.x] = o;
+            s_dst[threadIdx.x] = next_slot(A, s_off, o, m, A.start_local[m.k]);
+        }
+    } else if (threadIdx.x < w.count) {
+        const uint32_t i = (uint32_t)w.first + threadIdx.x;
+        s_src[threadIdx.x] = A.perm[i];
+        s_dst[threadIdx.x] = i;
     }
     __syncthreads();
     const uint32_t rr = threadIdx.x % R.rpb, v = threadIdx.x / R.rpb;
@@ -912,7 +923,6 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
     if (active) {
         const uint32_t id = src.id[o];
         if (INTEGRATE) {
-            const uint64_t t = A.ctrl->step - 1;
             const Ring rg = ring_at(t, sa.cap, sa.newest_first);
             auto pos = [&](int i, int k) { return src.pos[(uint64_t)(i * D + k) * N + o]; };
             auto vel = [&](int i, int k) { return src.vel[(uint64_t)(i * D + k) * N + o]; };
@@ -1073,12 +1083,14 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
                 const int ax = k + 3 - D;
                 ok = ok && axis_index(c1[k] / (double)nv, P.min[ax], P.dx[ax], P.n[ax], idx[ax]);
             }
-            uint32_t key = dst.vox[s];
+            uint32_t key = A.key[o];
             if (ok) key = P.voxel_offset + (idx[0] * P.n[1] + idx[1]) * P.n[2] + idx[2];
             else atomicAdd((unsigned long long*)&A.ctrl->out_of_grid, 1ull);
             A.key_next[s] = key;
+            note_move(A.delta, A.head_next, A.link_next, (uint32_t)s, A.key[o], key);
         }
     }
+    if constexpr (INTEGRATE) finish_order(A, s_off, sl0, t);
 }
 
 }  // namespace crm

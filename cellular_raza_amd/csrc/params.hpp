@@ -81,8 +81,11 @@ struct Control {
     uint32_t error_flags;   // bit (1 << crm_status) per error kind seen
     uint32_t n_div;         // rods dividing in the current step (cycle)
     uint64_t out_of_grid;   // agents that kept their voxel because the new index had no voxel
-    uint32_t skip;          // set by k_scan_local / k_sort_small: this step's sort is skipped (an earlier step failed)
+    uint32_t skip;          // set by k_scan_local / k_sort_small: this set-up sort is skipped (a step failed)
     uint32_t pad;
+    // `step` as the step's scan found it: what the gather reads, while one of its
+    // workgroups advances `step`
+    uint64_t gather_step;
     // index of the last step of the running crm_step call (or any earlier one): the
     // steps before it leave the ring entry that no later step reads unwritten
     uint64_t last_step;

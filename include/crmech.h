@@ -489,8 +489,10 @@ crm_status crm_save_cells_json(crm_ctx* ctx, const char* path, uint64_t iteratio
  * reference).  The event pairs around the launches are recorded without waiting;
  * crm_get_timing waits for those still in flight and adds them in, and
  * crm_reset_timing does the same before clearing the sums.  A class may cover
- * several launches per step (the scans, or all three sort kernels when the voxels
- * fit one scan tile, count as CRM_KERNEL_SCAN). */
+ * several launches (a set-up's scans, or all three sort kernels when the voxels fit
+ * one scan tile, count as CRM_KERNEL_SCAN).  A step of a timed context launches the
+ * scan of the next order (CRM_KERNEL_SCAN) and its voxel starts (CRM_KERNEL_SCATTER) on
+ * their own; other contexts do both inside the force and gather kernels. */
 crm_status crm_get_timing(crm_ctx* ctx, crm_timing* timing);
 crm_status crm_reset_timing(crm_ctx* ctx);
 
