@@ -620,8 +620,8 @@ __device__ __forceinline__ void rod_bend_window(const InstParams& P, Pos pos, in
     }
 }
 
-// LDS of the bending windows of a workgroup's rods: lane t holds window v of its
-// rod (t = lane of vertex v), read by the lanes of vertices v, v + 1, v + 2.
+// LDS of the bending windows of a workgroup's rods in the cycle's kernel: lane t holds
+// window v of its rod (t = lane of vertex v), read by the lanes of vertices v, v + 1, v + 2.
 constexpr int kRodWinK = kBlock * 3;
 
 // RodMechanics::calculate_increment row v (bacterial_rods.rs:157-213): springs,
@@ -868,104 +868,115 @@ __device__ __forceinline__ void rod_ahead(const InstParams& P, const StepArgs& s
 // position update needs neither the force nor noise other than the next step's
 // (Philox, or none), so the new vertex positions, velocities and ring give the
 // next centroid; the step's boundary error is raised here then.
+//
+// Latency-bound (1.6 KB and a chain of dependent loads per rod): every lane loads its own
+// row of the state once, before anything waits, and the rows of its neighbours come from
+// LDS, where row q, component k of rod r is word (q * D + k) * rp + r, rp odd, so that
+// neither a row nor a rod's rows meet in one bank.  200,000 2-D rods of 8 vertices 118 ->
+// 89 us, 12,347 in FP64 18.9 -> 16.0 (rows from global memory, several times each, after the slots).
+constexpr int kRodRows = kBlock * 3 + 48;  // 16 vertices, 3-D: 48 rows of 17 words
 template <int D, bool INTEGRATE, bool AHEAD>
 __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, StateBuf dst, RodArgs R,
                                                          StepArgs sa) {
-    __shared__ double newpos[kRodLdsK];
-    __shared__ double win[INTEGRATE ? kRodWinK : 1];
-    __shared__ double aheadpos[AHEAD ? kRodLdsK : 1];
+    __shared__ double newpos[kRodRows];
+    __shared__ double win[INTEGRATE ? kRodRows : 1];
+    __shared__ double aheadpos[AHEAD ? kRodRows : 1];
     __shared__ uint32_t s_off[INTEGRATE ? kStepScanTiles : 1];
+    __shared__ uint32_t s_src[INTEGRATE ? 1 : kBlock], s_dst[kBlock];
     const uint64_t t = INTEGRATE ? A.ctrl->gather_step : 0u;
-    if (INTEGRATE ? halted(A.ctrl, t) : A.ctrl->skip != 0u) return;
     const BlockWork w = A.work[blockIdx.x];
+    if (INTEGRATE ? halted(A.ctrl, t) : A.ctrl->skip != 0u) return;
     const uint32_t nv = R.nv, K = nv * D;
     // rods fastest across the lanes: thread t takes vertex row t / rpb of the
     // block's rod t % rpb, so that a wave's loads and stores of one component row
-    // cover consecutive slots.  lt = rod * nv + vertex addresses the LDS rows.  The
-    // streams read or written once (forces, the new state and ring) bypass the
-    // caches' retention (nontemporal; 200,000 2-D rods 125 -> 118 us); positions stay cached, the
-    // neighbouring vertex rows read them again.
-    __shared__ uint32_t s_src[kBlock], s_dst[kBlock];
-    uint32_t sl0 = 0;
-    if constexpr (INTEGRATE) {
-        const Move m = move_of(A, src.vox, (uint32_t)w.first, w.count);
-        sl0 = first_start_local(A);
-        step_tile_offsets(A, s_off);
-        if (threadIdx.x < w.count) {
-            const uint32_t o = (uint32_t)w.first + threadIdx.x;
-            s_src[threadIdx.x] = o;
-            s_dst[threadIdx.x] = next_slot(A, s_off, o, m, A.start_local[m.k]);
-        }
-    } else if (threadIdx.x < w.count) {
-        const uint32_t i = (uint32_t)w.first + threadIdx.x;
-        s_src[threadIdx.x] = A.perm[i];
-        s_dst[threadIdx.x] = i;
-    }
-    __syncthreads();
-    const uint32_t rr = threadIdx.x % R.rpb, v = threadIdx.x / R.rpb;
+    // cover consecutive slots.  The streams read or written once bypass the caches'
+    // retention (nontemporal; 200,000 2-D rods 125 -> 118 us).
+    const uint32_t rr = threadIdx.x % R.rpb, v = threadIdx.x / R.rpb, rp = R.rpb | 1u;
     const bool active = v < nv && rr < w.count;
-    const uint32_t o = active ? s_src[rr] : 0u;
-    const uint64_t s = active ? s_dst[rr] : 0u;
-    const uint32_t lt = rr * nv + v;
+    auto cell = [&](int q, int k) -> uint32_t { return (uint32_t)(q * D + k) * rp + rr; };
     const InstParams& P = A.ip[w.inst];
     const uint64_t N = A.N;
+    uint32_t o = (uint32_t)w.first + rr, id = 0, sl0 = 0;
+    const Ring rg = ring_at(t, sa.cap, sa.newest_first);
     double nx[D], nvel[D];
-    if constexpr (INTEGRATE) {  // bending window v of the rod, shared with the next two lanes
-        if (active && v + 2 < nv) {
-            auto pos = [&](int i, int k) { return src.pos[(uint64_t)(i * D + k) * N + o]; };
+    if constexpr (INTEGRATE) {
+        const Move m = move_of(A, src.vox, (uint32_t)w.first, w.count);
+        const uint32_t sl = threadIdx.x < w.count ? A.start_local[m.k] : 0u;
+        sl0 = first_start_local(A);
+        // own row, and the ring's other slot (capacity 2, filled from step 1 on), the only
+        // one that is read besides the slot written now
+        const bool older = rg.cap == 2 && t > 0;
+        const uint32_t h_old = 1u - rg.wslot;
+        double x[D], vv[D], f[D], hx[D], hv[D], dx[D], dv[D], dxr[D], spring = 0.0;
+        if (active) {
+            id = src.id[o];
+            spring = src.spring[o];
+#pragma unroll
+            for (int k = 0; k < D; k++) {
+                const uint64_t e = (uint64_t)(v * D + k) * N + o, eh = e + (uint64_t)h_old * K * N;
+                x[k] = __builtin_nontemporal_load(&src.pos[e]);
+                vv[k] = __builtin_nontemporal_load(&src.vel[e]);
+                f[k] = __builtin_nontemporal_load(&A.force[e]);
+                hx[k] = older ? __builtin_nontemporal_load(&src.hdx[eh]) : 0.0;
+                hv[k] = older ? __builtin_nontemporal_load(&src.hdv[eh]) : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < D; k++) newpos[cell((int)v, k)] = x[k];
+        }
+        step_tile_offsets(A, s_off);
+        if (threadIdx.x < w.count) s_dst[threadIdx.x] = next_slot(A, s_off, (uint32_t)w.first + threadIdx.x, m, sl);
+        auto pos = [&](int i, int k) { return newpos[cell(i, k)]; };
+        if (active && v + 2 < nv) {  // bending window v of the rod, shared with the next two lanes
             double F[D];
             rod_bend_window<D>(P, pos, (int)v, F);
 #pragma unroll
-            for (int k = 0; k < D; k++) win[lt * 3 + k] = F[k];
+            for (int k = 0; k < D; k++) win[cell((int)v, k)] = F[k];
         }
         __syncthreads();
-    }
-    if (active) {
-        const uint32_t id = src.id[o];
-        if (INTEGRATE) {
-            const Ring rg = ring_at(t, sa.cap, sa.newest_first);
-            auto pos = [&](int i, int k) { return src.pos[(uint64_t)(i * D + k) * N + o]; };
-            auto vel = [&](int i, int k) { return src.vel[(uint64_t)(i * D + k) * N + o]; };
-            double x[D], vv[D], f[D], dx[D], dv[D], dxr[D];
-#pragma unroll
-            for (int k = 0; k < D; k++) {
-                x[k] = pos((int)v, k);
-                vv[k] = vel((int)v, k);
-                f[k] = __builtin_nontemporal_load(&A.force[(uint64_t)(v * D + k) * N + o]);
-            }
-            auto wn = [&](int i, int k) { return win[(lt - v + (uint32_t)i) * 3 + k]; };
-            rod_row_increment<D>(P, src.spring[o], nv, v, pos, vel, wn, f, dx, dv);
+        if (active) {
+            auto wn = [&](int i, int k) { return win[cell(i, k)]; };
+            auto vel = [&](int, int k) { return vv[k]; };  // (only the own row's is asked for)
+            rod_row_increment<D>(P, spring, nv, v, pos, vel, wn, f, dx, dv);
             rod_row_noise<D>(P, sa, id, t, nv, v, dxr);
-            auto hist = [&](int i, int k, bool is_dv) {
-                const double* h = is_dv ? src.hdv : src.hdx;
-                return h[((uint64_t)rg.it[i] * K + v * D + k) * N + o];
-            };
+            auto hist = [&](int, int k, bool is_dv) { return is_dv ? hv[k] : hx[k]; };
             rod_row_solve<D, true>(sa, rg, x, vv, dx, dv, dxr, hist, nx, nvel);
             const bool out = rod_row_reflect<D, true>(P, nx, nvel);
             if (AHEAD && out) raise_error(A.ctrl, CRM_BOUNDARY_ERROR, t, id);
             if constexpr (AHEAD) {
-                // the ring after this step: slot rg.wslot holds dx, the others src's
-                const Ring rg1 = ring_at(t + 1, sa.cap, sa.newest_first);
-                auto hist1 = [&](int i, int k, bool) {
-                    const uint32_t sl = rg1.it[i];
-                    return sl == rg.wslot ? dx[k] : src.hdx[((uint64_t)sl * K + v * D + k) * N + o];
-                };
-                rod_ahead<D>(P, sa, t + 1, id, nv, v, nx, nvel, hist1, aheadpos + lt * 3);
-            }
-            if (rg.cap > 0) {
-                const uint32_t n_hist = (uint32_t)min<uint64_t>(t + 1, rg.cap);
-                const bool both = t >= A.ctrl->last_step;  // (see k_gather_integrate_point)
-                for (uint32_t h = 0; h < n_hist; h++) {
-                    if (h != rg.wslot && !both) continue;
+                // the next step's other slot is the one written now
+                auto hist1 = [&](int, int k, bool) { return dx[k]; };
+                double an[D];
+                rod_ahead<D>(P, sa, t + 1, id, nv, v, nx, nvel, hist1, an);
 #pragma unroll
-                    for (int k = 0; k < D; k++) {
-                        const uint64_t e = ((uint64_t)h * K + v * D + k) * N;
-                        __builtin_nontemporal_store(h == rg.wslot ? dx[k] : src.hdx[e + o], &dst.hdx[e + s]);
-                        __builtin_nontemporal_store(h == rg.wslot ? dv[k] : src.hdv[e + o], &dst.hdv[e + s]);
+                for (int k = 0; k < D; k++) aheadpos[cell((int)v, k)] = an[k];
+            }
+            const uint64_t s = s_dst[rr];
+            if (rg.cap > 0) {
+                const bool both = older && t >= A.ctrl->last_step;  // (see k_gather_integrate_point)
+#pragma unroll
+                for (int k = 0; k < D; k++) {
+                    const uint64_t e = (uint64_t)(v * D + k) * N + s;
+                    __builtin_nontemporal_store(dx[k], &dst.hdx[e + (uint64_t)rg.wslot * K * N]);
+                    __builtin_nontemporal_store(dv[k], &dst.hdv[e + (uint64_t)rg.wslot * K * N]);
+                    if (both) {
+                        __builtin_nontemporal_store(hx[k], &dst.hdx[e + (uint64_t)h_old * K * N]);
+                        __builtin_nontemporal_store(hv[k], &dst.hdv[e + (uint64_t)h_old * K * N]);
                     }
                 }
             }
-        } else {
+        }
+        __syncthreads();  // the old positions are read
+    } else {
+        if (threadIdx.x < w.count) {
+            const uint32_t i = (uint32_t)w.first + threadIdx.x;
+            s_src[threadIdx.x] = A.perm[i];
+            s_dst[threadIdx.x] = i;
+        }
+        __syncthreads();
+        if (active) {
+            o = s_src[rr];
+            id = src.id[o];
+            const uint64_t s = s_dst[rr];
             // every ring slot: rods born at different steps hold different counts
             const uint32_t n_hist = sa.cap;
 #pragma unroll
@@ -987,14 +998,20 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
                 auto hist1 = [&](int i, int k, bool) {
                     return src.hdx[((uint64_t)rg1.it[i] * K + v * D + k) * N + o];
                 };
-                rod_ahead<D>(P, sa, t1, id, nv, v, nx, nvel, hist1, aheadpos + lt * 3);
+                double an[D];
+                rod_ahead<D>(P, sa, t1, id, nv, v, nx, nvel, hist1, an);
+#pragma unroll
+                for (int k = 0; k < D; k++) aheadpos[cell((int)v, k)] = an[k];
             }
         }
+    }
+    const uint64_t s = active ? s_dst[rr] : 0u;
+    if (active) {
 #pragma unroll
         for (int k = 0; k < D; k++) {
             __builtin_nontemporal_store(nx[k], &dst.pos[(uint64_t)(v * D + k) * N + s]);
             __builtin_nontemporal_store(nvel[k], &dst.vel[(uint64_t)(v * D + k) * N + s]);
-            newpos[lt * 3 + k] = nx[k];
+            newpos[cell((int)v, k)] = nx[k];
         }
         if (v == 0) {
             dst.species[s] = src.species[o];
@@ -1007,16 +1024,15 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
     // the force records rec[slot][K] of the block's rods, a contiguous range but for
     // arrivals, written element by element from LDS
     for (uint32_t e = threadIdx.x; e < w.count * K; e += kBlock) {
-        const uint32_t r = e / K, c = e - r * K, vq = c / D;
-        R.rec[(uint64_t)s_dst[r] * K + c] = newpos[(r * nv + vq) * 3 + (c - vq * D)];
+        const uint32_t r = e / K, c = e - r * K;
+        R.rec[(uint64_t)s_dst[r] * K + c] = newpos[c * rp + r];
     }
     // the rod's vertex mean (every lane of the rod computes the same)
     auto mean = [&](double* c) {
-        const uint32_t l0 = rr * nv;
         c[0] = c[1] = c[2] = 0.0;
         for (uint32_t q = 0; q < nv; q++) {
 #pragma unroll
-            for (int k = 0; k < D; k++) c[k] = c[k] + newpos[(l0 + q) * 3 + k];
+            for (int k = 0; k < D; k++) c[k] = c[k] + newpos[cell((int)q, k)];
         }
 #pragma unroll
         for (int k = 0; k < D; k++) c[k] = c[k] / (double)nv;
@@ -1030,7 +1046,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
         bool zero = true;
 #pragma unroll
         for (int k = 0; k < D; k++) {
-            const double a = newpos[lt * 3 + k], b = newpos[(lt + 1) * 3 + k];
+            const double a = newpos[cell((int)v, k)], b = newpos[cell((int)v + 1, k)];
             o[k] = (float)((a + b) * 0.5 - c[k]);
             const float d = (float)(b - a);
             h2 = fmaf(d, d, h2);
@@ -1048,7 +1064,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
             double d2 = 0.0;
 #pragma unroll
             for (int k = 0; k < D; k++) {
-                const double d = newpos[(lt + q) * 3 + k] - c[k];
+                const double d = newpos[cell((int)q, k)] - c[k];
                 d2 = d2 + d * d;
             }
             r2 = fmax(r2, d2);
@@ -1061,7 +1077,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
             bool same = true;
 #pragma unroll
             for (int k = 0; k < D; k++)
-                same = same && newpos[(lt + q) * 3 + k] == newpos[(lt + q + 1) * 3 + k];
+                same = same && newpos[cell((int)q, k)] == newpos[cell((int)q + 1, k)];
             degenerate = degenerate || same;
         }
         // radius rounded up by a relative 1e-12 so that it covers every vertex
@@ -1074,7 +1090,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_rod(Arrays A, StateBuf src, S
             for (int k = 0; k < D; k++) c1[k] = 0.0;
             for (uint32_t q = 0; q < nv; q++) {
 #pragma unroll
-                for (int k = 0; k < D; k++) c1[k] = c1[k] + aheadpos[(lt + q) * 3 + k];
+                for (int k = 0; k < D; k++) c1[k] = c1[k] + aheadpos[cell((int)q, k)];
             }
             uint32_t idx[3] = {0, 0, 0};
             bool ok = true;
