@@ -1059,41 +1059,39 @@ crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
     return CRM_OK;
 }
 
-// A [C][N] array by slot (double, or the mixed path's float forces) to be read as
-// rows of C by agent index.
+// A [C][N] array by slot to be read as rows of C by agent index.
 struct RowRead {
     const void* src;
-    bool f32;
-    uint32_t C;
     double* out;
 };
 
-// Reads up to two arrays.  The rows are gathered on the device, for small systems
-// straight into pinned host memory, else into the other state buffer (free between
-// steps: every step writes it whole before it reads it) and copied out from there.
-crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n) {
+// Reads one or two arrays of C components (f32: of the mixed path's float forces, else
+// double).  The rows are gathered on the device, for small systems straight into pinned
+// host memory, else into the other state buffer (free between steps: every step writes
+// it whole before it reads it) and copied out from there.
+crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n, uint32_t C, bool f32 = false) {
     const uint64_t N = ctx->N;
-    size_t total = 0;
-    for (int i = 0; i < n; i++) total += (size_t)N * r[i].C * sizeof(double);
-    const bool small = total <= kPinDirect;
-    double* scratch[2] = {ctx->buf[1 - ctx->cur].pos, ctx->buf[1 - ctx->cur].vel};
-    HostPiece piece[2];
-    uint8_t* pin = ctx->pin + kPinControl;
-    for (int i = 0; i < n; i++) {
-        const size_t bytes = (size_t)N * r[i].C * sizeof(double);
-        double* dst = small ? reinterpret_cast<double*>(pin) : scratch[i];
-        piece[i] = HostPiece{reinterpret_cast<const uint8_t*>(dst), reinterpret_cast<uint8_t*>(r[i].out), bytes};
-        pin += bytes;
-        const dim3 g((uint32_t)((N + kBlock - 1) / kBlock)), b(kBlock);
-        const uint32_t* id = ctx->buf[ctx->cur].id;
-        if (r[i].f32)
-            hipLaunchKernelGGL(k_rows_by_id<float>, g, b, 0, ctx->stream, static_cast<const float*>(r[i].src), id, dst,
-                               N, r[i].C);
-        else
-            hipLaunchKernelGGL(k_rows_by_id<double>, g, b, 0, ctx->stream, static_cast<const double*>(r[i].src), id,
-                               dst, N, r[i].C);
-        CRM_HIP(hipGetLastError());
+    const size_t bytes = (size_t)N * C * sizeof(double);
+    const bool small = n * bytes <= kPinDirect;
+    uint8_t* const pin = ctx->pin + kPinControl;
+    double* dst[2] = {ctx->buf[1 - ctx->cur].pos, ctx->buf[1 - ctx->cur].vel};
+    if (small) {
+        dst[0] = reinterpret_cast<double*>(pin);
+        dst[1] = reinterpret_cast<double*>(pin + bytes);
     }
+    HostPiece piece[2];
+    for (int i = 0; i < n; i++)
+        piece[i] = HostPiece{reinterpret_cast<const uint8_t*>(dst[i]), reinterpret_cast<uint8_t*>(r[i].out), bytes};
+    const void *src0 = r[0].src, *src1 = r[n - 1].src;
+    const dim3 g((uint32_t)((N + kBlock - 1) / kBlock), (uint32_t)n), b(kBlock);
+    const uint32_t* id = ctx->buf[ctx->cur].id;
+    if (f32)
+        hipLaunchKernelGGL(k_rows_by_id<float>, g, b, 0, ctx->stream, static_cast<const float*>(src0),
+                           static_cast<const float*>(src1), id, dst[0], dst[1], N, C);
+    else
+        hipLaunchKernelGGL(k_rows_by_id<double>, g, b, 0, ctx->stream, static_cast<const double*>(src0),
+                           static_cast<const double*>(src1), id, dst[0], dst[1], N, C);
+    CRM_HIP(hipGetLastError());
     if (!small) return copy_out(ctx, piece, n);
     CRM_HIP(hipStreamSynchronize(ctx->stream));
     for (int i = 0; i < n; i++) std::memcpy(piece[i].host, piece[i].dev, piece[i].bytes);
@@ -2297,8 +2295,8 @@ crm_status crm_compute_forces(crm_ctx* ctx, double* force) {
     CRM_HIP(hipSetDevice(ctx->device));
     CRM_TRY(launch_force(ctx));
     CRM_TRY(check_errors(ctx, "forces"));
-    const RowRead r{ctx->d_force, force_f32(ctx), ctx->K, force};
-    return read_rows(ctx, &r, 1);
+    const RowRead r{ctx->d_force, force};
+    return read_rows(ctx, &r, 1, ctx->K, force_f32(ctx));
 }
 
 crm_status crm_get_state(crm_ctx* ctx, double* pos, double* vel) {
@@ -2307,9 +2305,9 @@ crm_status crm_get_state(crm_ctx* ctx, double* pos, double* vel) {
     const StateBuf& S = ctx->buf[ctx->cur];
     RowRead r[2];
     int n = 0;
-    if (pos) r[n++] = RowRead{S.pos, false, ctx->K, pos};
-    if (vel) r[n++] = RowRead{S.vel, false, ctx->K, vel};
-    return n ? read_rows(ctx, r, n) : CRM_OK;
+    if (pos) r[n++] = RowRead{S.pos, pos};
+    if (vel) r[n++] = RowRead{S.vel, vel};
+    return n ? read_rows(ctx, r, n, ctx->K) : CRM_OK;
 }
 
 crm_status crm_get_history(crm_ctx* ctx, double* dx_hist, double* dv_hist, uint32_t* n_stored) {
@@ -2357,9 +2355,9 @@ crm_status crm_get_history(crm_ctx* ctx, double* dx_hist, double* dv_hist, uint3
             RowRead r[2];
             int n = 0;
             const StateBuf& S = ctx->buf[ctx->cur];
-            if (dx_hist) r[n++] = RowRead{S.hdx + slot * slot_elems, false, ctx->K, dx_hist + i * slot_elems};
-            if (dv_hist) r[n++] = RowRead{S.hdv + slot * slot_elems, false, ctx->K, dv_hist + i * slot_elems};
-            if (n) CRM_TRY(read_rows(ctx, r, n));
+            if (dx_hist) r[n++] = RowRead{S.hdx + slot * slot_elems, dx_hist + i * slot_elems};
+            if (dv_hist) r[n++] = RowRead{S.hdv + slot * slot_elems, dv_hist + i * slot_elems};
+            if (n) CRM_TRY(read_rows(ctx, r, n, ctx->K));
         } else {
             if (dx_hist) std::fill(dx_hist + i * slot_elems, dx_hist + (i + 1) * slot_elems, 0.0);
             if (dv_hist) std::fill(dv_hist + i * slot_elems, dv_hist + (i + 1) * slot_elems, 0.0);
@@ -2597,12 +2595,12 @@ crm_status crm_get_cycle_state(crm_ctx* ctx, double* spring_length, double* grow
     const uint64_t N = ctx->N;
     const StateBuf& S = ctx->buf[ctx->cur];
     if (spring_length) {
-        const RowRead r{S.spring, false, 1, spring_length};
-        CRM_TRY(read_rows(ctx, &r, 1));
+        const RowRead r{S.spring, spring_length};
+        CRM_TRY(read_rows(ctx, &r, 1, 1));
     }
     if (growth_rate) {
-        const RowRead r{S.growth, false, 1, growth_rate};
-        CRM_TRY(read_rows(ctx, &r, 1));
+        const RowRead r{S.growth, growth_rate};
+        CRM_TRY(read_rows(ctx, &r, 1, 1));
     }
     std::vector<uint64_t> tmp(3 * N);
     uint64_t* outs[2] = {identifier, parent};

@@ -62,12 +62,16 @@ __global__ __launch_bounds__(kBlock) void k_snapshot(StateBuf S, SnapshotArgs a)
 // Rows by agent index from a [C][N] array by slot.  Thread per slot: the reads of a
 // component are coalesced, a thread's row is written by consecutive stores that
 // merge in L2.
+// blockIdx.y picks one of two arrays: a read of positions and velocities is one launch
+// (1000 agents, step and read: 50.0 -> 47.9 us).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_rows_by_id(const T* __restrict__ src, const uint32_t* __restrict__ id,
-                                                        double* __restrict__ out, uint64_t N, uint32_t C) {
+__global__ __launch_bounds__(kBlock) void k_rows_by_id(const T* __restrict__ src0, const T* __restrict__ src1,
+                                                        const uint32_t* __restrict__ id, double* __restrict__ out0,
+                                                        double* __restrict__ out1, uint64_t N, uint32_t C) {
     const uint64_t s = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (s >= N) return;
-    double* o = out + (uint64_t)id[s] * C;
+    const T* src = blockIdx.y ? src1 : src0;
+    double* o = (blockIdx.y ? out1 : out0) + (uint64_t)id[s] * C;
     for (uint32_t k = 0; k < C; k++) o[k] = (double)src[(uint64_t)k * N + s];
 }
 
