@@ -196,8 +196,8 @@ constexpr size_t kPinDirect = 256 * 1024;
 constexpr uint64_t kNoAllocMaxAgents = 1ull << 22;
 constexpr uint32_t kNoAllocMaxInstances = 1u << 16;
 constexpr size_t kNoAllocScanReserve = (size_t)1 << 20;
-// Steps per long graph replay (even, so that a replay keeps the buffer parity).
-constexpr uint32_t kLongGraphSteps = 16;
+// Steps per graph replay (even, so that a replay keeps the buffer parity).
+constexpr uint32_t kGraphSteps = 16;
 // Steps of a call from which the carry of the older ring entry is left to the last one.
 constexpr uint32_t kCarryLastSteps = 8;
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -303,9 +303,8 @@ struct crm_ctx {
     bool halted = false;
     uint64_t step = 0;
 
-    // graphs for the two buffer parities: [parity] replays two steps, [2 + parity]
-    // kLongGraphSteps steps
-    hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
+    // a graph of kGraphSteps steps for each buffer parity
+    hipGraphExec_t graph[2] = {nullptr, nullptr};
 
     // timing: an event pair around each launch (class t_cls[i]), recorded without
     // waiting, so that the timed kernels run back to back as in a normal step;
@@ -1106,14 +1105,14 @@ crm_status download_ids(crm_ctx* ctx, std::vector<uint32_t>& id) {
     return CRM_OK;
 }
 
-crm_status build_graph(crm_ctx* ctx, int parity, bool long_graph) {
+crm_status build_graph(crm_ctx* ctx, int parity) {
     // An even number of steps returns the buffers to the same parity, so one
-    // captured sequence of two (or kLongGraphSteps) steps replays from either parity.
+    // captured sequence of kGraphSteps steps replays from the parity it was built for.
     int saved = ctx->cur;
     ctx->cur = parity;
     CRM_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     crm_status st = CRM_OK;
-    for (uint32_t k = 0; k < (long_graph ? kLongGraphSteps : 2u) && st == CRM_OK; k++) st = launch_step(ctx, nullptr);
+    for (uint32_t k = 0; k < kGraphSteps && st == CRM_OK; k++) st = launch_step(ctx, nullptr);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     ctx->cur = saved;
@@ -1125,7 +1124,7 @@ crm_status build_graph(crm_ctx* ctx, int parity, bool long_graph) {
         ctx->err = std::string("HIP error: ") + hipGetErrorString(e) + " at hipStreamEndCapture";
         return CRM_DEVICE_ERROR;
     }
-    e = hipGraphInstantiate(&ctx->graph[(long_graph ? 2 : 0) + parity], g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&ctx->graph[parity], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) {
         ctx->err = std::string("HIP error: ") + hipGetErrorString(e) + " at hipGraphInstantiate";
@@ -2248,16 +2247,15 @@ crm_status crm_step(crm_ctx* ctx, uint32_t n_steps, const double* noise) {
         CRM_HIP(hipGetLastError());
     }
     uint32_t s = 0;
-    if (graphs) {  // each graph launch costs the device a few microseconds
-        while (s + kLongGraphSteps <= n_steps) {
-            if (!ctx->graph[2 + ctx->cur]) CRM_TRY(build_graph(ctx, ctx->cur, true));
-            CRM_HIP(hipGraphLaunch(ctx->graph[2 + ctx->cur], ctx->stream));
-            s += kLongGraphSteps;
-        }
-        while (s + 2 <= n_steps) {
-            if (!ctx->graph[ctx->cur]) CRM_TRY(build_graph(ctx, ctx->cur, false));
+    // Whole graphs only: a graph launch costs the device about 9 us, more than the rest's two
+    // launches a step, which the host queues faster than the kernels run (two-step graphs
+    // for the rest: short run of 2 x 10 steps 1.51 -> 1.38 ms without them, which also saves
+    // building them, 50 steps of 30,000 agents 1.36 -> 1.30)
+    if (graphs) {
+        while (s + kGraphSteps <= n_steps) {
+            if (!ctx->graph[ctx->cur]) CRM_TRY(build_graph(ctx, ctx->cur));
             CRM_HIP(hipGraphLaunch(ctx->graph[ctx->cur], ctx->stream));
-            s += 2;
+            s += kGraphSteps;
         }
     }
     for (; s < n_steps; s++) CRM_TRY(launch_step(ctx, use_noise_buf ? ctx->d_noise + per_step * s : nullptr));
