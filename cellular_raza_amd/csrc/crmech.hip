@@ -167,24 +167,25 @@ static void fill_pot(PotParams<T>& q, const crm_potential& p) {
 enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 
 // ---- host transfers ---------------------------------------------------------
-// Each context owns a pinned block: the control block's copy, then kPinWorkers
-// chunks of kPinChunkSmall bytes.  Read-backs of small systems are written there by
-// the gathering kernel; larger ones are copied out chunk by chunk, each chunk emptied
-// by a host thread of its own: one thread fills fresh pages of the caller's array at
-// 4.5 GB/s (page faults), two at 8, four at 12.5, eight at 19-20 GB/s (48 MB and
-// 192 MB; the link carries 55 GB/s).  Read-backs above kPinLarge get kPinChunkLarge
-// chunks, allocated on the first one (48 MB: 2.7 ms in either size, 192 MB: 9.9 ms
-// against 10.9 with half of it; 8 MB: 0.59 against 0.76 ms in small chunks); an
-// allocation takes 0.1 ms up to 2 MB, 0.3 ms at 8.
+// Each context owns a pinned block: the control block's copy, then room for a read-back
+// of kPinDirect bytes.  Read-backs up to there are written to it by the gathering kernel
+// itself and moved on in parts of kPinPart bytes by a host thread for every whole
+// kPinPerThread of them; larger ones are copied out through kPinWorkers chunks of kPinChunk bytes
+// (allocated on the first one), each queued, awaited and emptied by a host thread of its
+// own: one thread fills fresh pages of the caller's array at 4.5 GB/s (page faults), two
+// at 8, four at 12.5, eight at 19-20 GB/s (48 MB and 192 MB; the link carries 55 GB/s).
+// The lines lie where both sides meet: threads that call HIP cost 20 us more than ones
+// that copy (get_state of 516 KB 98 us with two of them, 52 with the kernel's own stores
+// and none), a second thread pays from 1 MB on (0.5 MB to a thread: forces of 90,000
+// agents, 2.1 MB, 217 us with four, 237 with one, 240 with eight), and above 2 MB the copies
+// overlap the moves (get_state of 2.9 MB 163 us in chunks of 1 MB, 208 in ones of 0.5, 222
+// by the kernel's stores).
 constexpr size_t kPinControl = 4096;
 constexpr uint32_t kPinWorkers = 8;
-constexpr size_t kPinChunkSmall = 256 * 1024;
-constexpr size_t kPinChunkLarge = 1024 * 1024;
-constexpr size_t kPinLarge = 4 * 1024 * 1024;
-// Largest read-back that the kernel writes to pinned memory itself: get_state takes
-// 36 us at 259 KB, and 94 us at 269 KB through two host threads (256 KB and more to a
-// thread is where a second one pays for its start).
-constexpr size_t kPinDirect = 256 * 1024;
+constexpr size_t kPinDirect = 2 * 1024 * 1024;
+constexpr size_t kPinPerThread = 512 * 1024;
+constexpr size_t kPinPart = 256 * 1024;
+constexpr size_t kPinChunk = 1024 * 1024;
 
 // ---- device scratch of crm_remove_agents_noalloc ---------------------------
 // One static array per GPU, sized for kNoAllocMaxAgents agents in at most
@@ -316,8 +317,8 @@ struct crm_ctx {
     double t_ms[CRM_KERNEL_COUNT] = {};
     uint64_t t_n[CRM_KERNEL_COUNT] = {};
 
-    uint8_t* pin = nullptr;        // kPinControl bytes + kPinWorkers chunks of kPinChunkSmall
-    uint8_t* pin_large = nullptr;  // kPinWorkers chunks of kPinChunkLarge
+    uint8_t* pin = nullptr;         // kPinControl + kPinDirect bytes
+    uint8_t* pin_chunks = nullptr;  // kPinWorkers chunks of kPinChunk
     hipEvent_t pin_ev[kPinWorkers] = {};
 };
 
@@ -1004,58 +1005,81 @@ struct HostPiece {
     size_t bytes;
 };
 
-// Copies the pieces to pageable host memory, chunk by chunk through pinned memory:
-// every host thread takes the next chunk, queues its copy into its own pinned chunk
-// and moves it on once it has arrived.  The stream's earlier work precedes the copies.
-crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
-    size_t total = 0;
-    for (int i = 0; i < n_pieces; i++) total += pieces[i].bytes;
-    const bool large = total > kPinLarge;
-    if (large && !ctx->pin_large)
-        CRM_HIP(hipHostMalloc((void**)&ctx->pin_large, kPinWorkers * kPinChunkLarge, hipHostMallocDefault));
-    uint8_t* const pins = large ? ctx->pin_large : ctx->pin + kPinControl;
-    const size_t chunk = large ? kPinChunkLarge : kPinChunkSmall;
-    size_t n_chunks = 0;
-    for (int i = 0; i < n_pieces; i++) n_chunks += (pieces[i].bytes + chunk - 1) / chunk;
-    const uint32_t hw = std::max(1u, std::thread::hardware_concurrency() / 2);
-    const uint32_t workers = (uint32_t)std::min<size_t>(std::min(kPinWorkers, hw), std::max<size_t>(n_chunks, 1));
-    for (uint32_t w = 0; w < workers; w++)
-        if (!ctx->pin_ev[w]) CRM_HIP(hipEventCreateWithFlags(&ctx->pin_ev[w], hipEventDisableTiming));
-    std::atomic<size_t> next{0};
-    std::atomic<int> failed{(int)hipSuccess};
-    auto work = [&](uint32_t w) {
-        hipError_t e = hipSetDevice(ctx->device);
-        uint8_t* const pin = pins + w * chunk;
-        while (e == hipSuccess && failed.load() == (int)hipSuccess) {
-            size_t c = next.fetch_add(1);
-            int i = 0;
-            for (; i < n_pieces; i++) {
-                const size_t nc = (pieces[i].bytes + chunk - 1) / chunk;
-                if (c < nc) break;
-                c -= nc;
-            }
-            if (i == n_pieces) return;
-            const size_t off = c * chunk, len = std::min(chunk, pieces[i].bytes - off);
-            e = hipMemcpyAsync(pin, pieces[i].dev + off, len, hipMemcpyDeviceToHost, ctx->stream);
-            if (e == hipSuccess) e = hipEventRecord(ctx->pin_ev[w], ctx->stream);
-            if (e == hipSuccess) e = hipEventSynchronize(ctx->pin_ev[w]);
-            if (e == hipSuccess) std::memcpy(pieces[i].host + off, pin, len);
-        }
-        if (e != hipSuccess) failed.store((int)e);
-    };
+// Calls work(w) for w < workers, each in a host thread of its own (w = 0 in this one).
+// Fewer run where no more threads are to be had: the work is shared out as it goes.
+template <typename Work>
+void on_threads(uint32_t workers, const Work& work) {
     std::thread threads[kPinWorkers];
     for (uint32_t w = 1; w < workers; w++) {
         try {
-            threads[w] = std::thread(work, w);
-        } catch (...) {  // no more threads to be had: the ones running share the chunks
+            threads[w] = std::thread([&work, w] { work(w); });
+        } catch (...) {
             break;
         }
     }
     work(0);
     for (auto& t : threads)
         if (t.joinable()) t.join();
+}
+
+uint32_t host_threads(size_t most) {
+    if (most <= 1) return 1;  // (asking for the number of CPUs takes 1 us)
+    const size_t hw = std::max(1u, std::thread::hardware_concurrency() / 2);
+    return (uint32_t)std::min(std::min<size_t>(kPinWorkers, hw), most);
+}
+
+// The c-th part of at most `part` bytes of the pieces (bytes = 0: there are no more).
+HostPiece piece_part(const HostPiece* pieces, int n_pieces, size_t part, size_t c) {
+    for (int i = 0; i < n_pieces; i++) {
+        const size_t nc = (pieces[i].bytes + part - 1) / part, off = c * part;
+        if (c < nc) return HostPiece{pieces[i].dev + off, pieces[i].host + off, std::min(part, pieces[i].bytes - off)};
+        c -= nc;
+    }
+    return HostPiece{nullptr, nullptr, 0};
+}
+
+// Copies the pieces to pageable host memory, chunk by chunk through pinned memory:
+// every host thread takes the next chunk, queues its copy into its own pinned chunk
+// and moves it on once it has arrived.  The stream's earlier work precedes the copies.
+crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
+    if (!ctx->pin_chunks)
+        CRM_HIP(hipHostMalloc((void**)&ctx->pin_chunks, kPinWorkers * kPinChunk, hipHostMallocDefault));
+    size_t n_chunks = 0;
+    for (int i = 0; i < n_pieces; i++) n_chunks += (pieces[i].bytes + kPinChunk - 1) / kPinChunk;
+    const uint32_t workers = host_threads(n_chunks);
+    for (uint32_t w = 0; w < workers; w++)
+        if (!ctx->pin_ev[w]) CRM_HIP(hipEventCreateWithFlags(&ctx->pin_ev[w], hipEventDisableTiming));
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    on_threads(workers, [&](uint32_t w) {
+        hipError_t e = hipSetDevice(ctx->device);
+        uint8_t* const pin = ctx->pin_chunks + w * kPinChunk;
+        while (e == hipSuccess && failed.load() == (int)hipSuccess) {
+            const HostPiece q = piece_part(pieces, n_pieces, kPinChunk, next.fetch_add(1));
+            if (!q.bytes) return;
+            e = hipMemcpyAsync(pin, q.dev, q.bytes, hipMemcpyDeviceToHost, ctx->stream);
+            if (e == hipSuccess) e = hipEventRecord(ctx->pin_ev[w], ctx->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(ctx->pin_ev[w]);
+            if (e == hipSuccess) std::memcpy(q.host, pin, q.bytes);
+        }
+        if (e != hipSuccess) failed.store((int)e);
+    });
     CRM_HIP((hipError_t)failed.load());
     return CRM_OK;
+}
+
+// Moves the pieces on from pinned memory, all of them written.
+void move_out(const HostPiece* pieces, int n_pieces) {
+    size_t total = 0;
+    for (int i = 0; i < n_pieces; i++) total += pieces[i].bytes;
+    std::atomic<size_t> next{0};
+    on_threads(host_threads(total / kPinPerThread), [&](uint32_t) {
+        for (;;) {
+            const HostPiece q = piece_part(pieces, n_pieces, kPinPart, next.fetch_add(1));
+            if (!q.bytes) return;
+            std::memcpy(q.host, q.dev, q.bytes);
+        }
+    });
 }
 
 // A [C][N] array by slot to be read as rows of C by agent index.
@@ -1065,16 +1089,16 @@ struct RowRead {
 };
 
 // Reads one or two arrays of C components (f32: of the mixed path's float forces, else
-// double).  The rows are gathered on the device, for small systems straight into pinned
+// double).  The rows are gathered on the device, up to kPinDirect straight into pinned
 // host memory, else into the other state buffer (free between steps: every step writes
 // it whole before it reads it) and copied out from there.
 crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n, uint32_t C, bool f32 = false) {
     const uint64_t N = ctx->N;
     const size_t bytes = (size_t)N * C * sizeof(double);
-    const bool small = n * bytes <= kPinDirect;
+    const bool direct = n * bytes <= kPinDirect;
     uint8_t* const pin = ctx->pin + kPinControl;
     double* dst[2] = {ctx->buf[1 - ctx->cur].pos, ctx->buf[1 - ctx->cur].vel};
-    if (small) {
+    if (direct) {
         dst[0] = reinterpret_cast<double*>(pin);
         dst[1] = reinterpret_cast<double*>(pin + bytes);
     }
@@ -1091,9 +1115,9 @@ crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n, uint32_t C, bool f32
         hipLaunchKernelGGL(k_rows_by_id<double>, g, b, 0, ctx->stream, static_cast<const double*>(src0),
                            static_cast<const double*>(src1), id, dst[0], dst[1], N, C);
     CRM_HIP(hipGetLastError());
-    if (!small) return copy_out(ctx, piece, n);
+    if (!direct) return copy_out(ctx, piece, n);
     CRM_HIP(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < n; i++) std::memcpy(piece[i].host, piece[i].dev, piece[i].bytes);
+    move_out(piece, n);
     return CRM_OK;
 }
 
@@ -1998,7 +2022,7 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
     if (hipMalloc((void**)&ctx->d_ip, sizeof(InstParams) * n_instances) != hipSuccess ||
         hipMalloc((void**)&ctx->d_ctrl, sizeof(Control)) != hipSuccess)
         return fail(CRM_DEVICE_ERROR, "hipMalloc failed");
-    if (hipHostMalloc((void**)&ctx->pin, kPinControl + kPinWorkers * kPinChunkSmall, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc((void**)&ctx->pin, kPinControl + kPinDirect, hipHostMallocDefault) != hipSuccess)
         return fail(CRM_DEVICE_ERROR, "hipHostMalloc failed");
     e = hipMemcpy(ctx->d_ip, ctx->hparams.data(), sizeof(InstParams) * n_instances, hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipMemcpy: ") + hipGetErrorString(e));
@@ -2956,7 +2980,7 @@ void crm_destroy(crm_ctx* ctx) {
     if (ctx->d_ip) (void)hipFree(ctx->d_ip);
     if (ctx->d_ctrl) (void)hipFree(ctx->d_ctrl);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
-    if (ctx->pin_large) (void)hipHostFree(ctx->pin_large);
+    if (ctx->pin_chunks) (void)hipHostFree(ctx->pin_chunks);
     for (auto e : ctx->pin_ev)
         if (e) (void)hipEventDestroy(e);
     for (int i = 0; i < crm_ctx::kTimingPairs; i++) {
