@@ -167,12 +167,11 @@ static void fill_pot(PotParams<T>& q, const crm_potential& p) {
 enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 
 // ---- host transfers ---------------------------------------------------------
-// Each context owns a pinned block: the control block's copy, then room for a read-back
-// of kPinDirect bytes.  Read-backs up to there are written to it by the gathering kernel
-// itself and moved on in parts of kPinPart bytes by a host thread for every whole
-// kPinPerThread of them; larger ones are copied out through kPinWorkers chunks of kPinChunk bytes
-// (allocated on the first one), each queued, awaited and emptied by a host thread of its
-// own: one thread fills fresh pages of the caller's array at 4.5 GB/s (page faults), two
+// What goes to the host passes through pinned memory, a block of one of kPinBytes that the
+// call borrows (PinLease).  Read-backs up to kPinDirect are written there by the gathering
+// kernel itself and moved on in parts of kPinPart bytes by a host thread for every whole
+// kPinPerThread of them; larger ones are copied out through kPinWorkers chunks of kPinChunk
+// bytes, each queued, awaited and emptied by a host thread of its own: one thread fills fresh pages of the caller's array at 4.5 GB/s (page faults), two
 // at 8, four at 12.5, eight at 19-20 GB/s (48 MB and 192 MB; the link carries 55 GB/s).
 // The lines lie where both sides meet: threads that call HIP cost 20 us more than ones
 // that copy (get_state of 516 KB 98 us with two of them, 52 with the kernel's own stores
@@ -180,12 +179,13 @@ enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 // agents, 2.1 MB, 217 us with four, 237 with one, 240 with eight), and above 2 MB the copies
 // overlap the moves (get_state of 2.9 MB 163 us in chunks of 1 MB, 208 in ones of 0.5, 222
 // by the kernel's stores).
-constexpr size_t kPinControl = 4096;
 constexpr uint32_t kPinWorkers = 8;
-constexpr size_t kPinDirect = 2 * 1024 * 1024;
+constexpr uint32_t kPinSizes = 3;
+constexpr size_t kPinBytes[kPinSizes] = {512 * 1024, 2 * 1024 * 1024, 8 * 1024 * 1024};
+constexpr size_t kPinDirect = kPinBytes[1];
 constexpr size_t kPinPerThread = 512 * 1024;
 constexpr size_t kPinPart = 256 * 1024;
-constexpr size_t kPinChunk = 1024 * 1024;
+constexpr size_t kPinChunk = kPinBytes[2] / kPinWorkers;
 
 // ---- device scratch of crm_remove_agents_noalloc ---------------------------
 // One static array per GPU, sized for kNoAllocMaxAgents agents in at most
@@ -317,8 +317,6 @@ struct crm_ctx {
     double t_ms[CRM_KERNEL_COUNT] = {};
     uint64_t t_n[CRM_KERNEL_COUNT] = {};
 
-    uint8_t* pin = nullptr;         // kPinControl + kPinDirect bytes
-    uint8_t* pin_chunks = nullptr;  // kPinWorkers chunks of kPinChunk
     hipEvent_t pin_ev[kPinWorkers] = {};
 };
 
@@ -813,14 +811,74 @@ crm_status launch_step(crm_ctx* ctx, const double* noise_step) {
     return CRM_OK;
 }
 
+// The process's pinned blocks that no call is using, at most two of each size (21 MiB):
+// with 2 MiB, and 8 more after a large read, in every context, 24 contexts alive at once
+// took 110 us more to create each, and 170 more for their first read of 30,000 agents.
+// The last context to be destroyed frees them.
+struct PinPool {
+    std::mutex m;
+    uint64_t contexts = 0;
+    uint8_t* idle[kPinSizes][2] = {};
+};
+PinPool g_pins;
+
+// A block for the duration of a call, accessible to every device.  `settled`: the work
+// queued on the block is done; else the stream is waited for before another call may get it.
+struct PinLease {
+    uint8_t* p = nullptr;
+    uint32_t size = 0;
+    bool settled = false;
+    const hipStream_t stream;
+    explicit PinLease(const crm_ctx* ctx) : stream(ctx->stream) {}
+    PinLease(const PinLease&) = delete;
+    PinLease& operator=(const PinLease&) = delete;
+    hipError_t take(size_t bytes) {
+        while (kPinBytes[size] < bytes) size++;
+        {
+            std::lock_guard<std::mutex> lock(g_pins.m);
+            for (auto& q : g_pins.idle[size])
+                if (q && !p) std::swap(p, q);
+        }
+        return p ? hipSuccess : hipHostMalloc((void**)&p, kPinBytes[size], hipHostMallocPortable);
+    }
+    ~PinLease() {
+        if (!p) return;
+        if (!settled) (void)hipStreamSynchronize(stream);
+        {
+            std::lock_guard<std::mutex> lock(g_pins.m);
+            for (auto& q : g_pins.idle[size])
+                if (!q && p) std::swap(p, q);
+        }
+        if (p) (void)hipHostFree(p);
+    }
+};
+
+void pin_pool_enter() {
+    std::lock_guard<std::mutex> lock(g_pins.m);
+    g_pins.contexts++;
+}
+
+void pin_pool_leave() {
+    std::lock_guard<std::mutex> lock(g_pins.m);
+    if (--g_pins.contexts) return;
+    for (auto& of_size : g_pins.idle)
+        for (auto& q : of_size) {
+            if (q) (void)hipHostFree(q);
+            q = nullptr;
+        }
+}
+
 // The control block after everything queued so far: a one-thread kernel writes it
-// to the context's pinned page (launch and wait 11 us; a copy to pageable memory 24).
+// to pinned memory (launch and wait 11 us; a copy to pageable memory 24).
 crm_status read_control(crm_ctx* ctx, Control& c) {
+    PinLease pin(ctx);
+    CRM_HIP(pin.take(sizeof(Control)));
     hipLaunchKernelGGL(k_publish_control, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl,
-                       reinterpret_cast<Control*>(ctx->pin));
+                       reinterpret_cast<Control*>(pin.p));
     CRM_HIP(hipGetLastError());
     CRM_HIP(hipStreamSynchronize(ctx->stream));
-    std::memcpy(&c, ctx->pin, sizeof(Control));
+    pin.settled = true;
+    std::memcpy(&c, pin.p, sizeof(Control));
     return CRM_OK;
 }
 
@@ -1042,8 +1100,8 @@ HostPiece piece_part(const HostPiece* pieces, int n_pieces, size_t part, size_t 
 // every host thread takes the next chunk, queues its copy into its own pinned chunk
 // and moves it on once it has arrived.  The stream's earlier work precedes the copies.
 crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
-    if (!ctx->pin_chunks)
-        CRM_HIP(hipHostMalloc((void**)&ctx->pin_chunks, kPinWorkers * kPinChunk, hipHostMallocDefault));
+    PinLease pins(ctx);
+    CRM_HIP(pins.take(kPinWorkers * kPinChunk));
     size_t n_chunks = 0;
     for (int i = 0; i < n_pieces; i++) n_chunks += (pieces[i].bytes + kPinChunk - 1) / kPinChunk;
     const uint32_t workers = host_threads(n_chunks);
@@ -1053,7 +1111,7 @@ crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
     std::atomic<int> failed{(int)hipSuccess};
     on_threads(workers, [&](uint32_t w) {
         hipError_t e = hipSetDevice(ctx->device);
-        uint8_t* const pin = ctx->pin_chunks + w * kPinChunk;
+        uint8_t* const pin = pins.p + w * kPinChunk;
         while (e == hipSuccess && failed.load() == (int)hipSuccess) {
             const HostPiece q = piece_part(pieces, n_pieces, kPinChunk, next.fetch_add(1));
             if (!q.bytes) return;
@@ -1065,6 +1123,7 @@ crm_status copy_out(crm_ctx* ctx, const HostPiece* pieces, int n_pieces) {
         if (e != hipSuccess) failed.store((int)e);
     });
     CRM_HIP((hipError_t)failed.load());
+    pins.settled = true;
     return CRM_OK;
 }
 
@@ -1096,11 +1155,12 @@ crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n, uint32_t C, bool f32
     const uint64_t N = ctx->N;
     const size_t bytes = (size_t)N * C * sizeof(double);
     const bool direct = n * bytes <= kPinDirect;
-    uint8_t* const pin = ctx->pin + kPinControl;
+    PinLease pin(ctx);
     double* dst[2] = {ctx->buf[1 - ctx->cur].pos, ctx->buf[1 - ctx->cur].vel};
     if (direct) {
-        dst[0] = reinterpret_cast<double*>(pin);
-        dst[1] = reinterpret_cast<double*>(pin + bytes);
+        CRM_HIP(pin.take(n * bytes));
+        dst[0] = reinterpret_cast<double*>(pin.p);
+        dst[1] = reinterpret_cast<double*>(pin.p + bytes);
     }
     HostPiece piece[2];
     for (int i = 0; i < n; i++)
@@ -1117,6 +1177,7 @@ crm_status read_rows(crm_ctx* ctx, const RowRead* r, int n, uint32_t C, bool f32
     CRM_HIP(hipGetLastError());
     if (!direct) return copy_out(ctx, piece, n);
     CRM_HIP(hipStreamSynchronize(ctx->stream));
+    pin.settled = true;
     move_out(piece, n);
     return CRM_OK;
 }
@@ -1900,6 +1961,7 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
         return CRM_INVALID_ARGUMENT;
     }
     crm_ctx* ctx = new crm_ctx();
+    pin_pool_enter();
     ctx->cfg = *cfg;
     auto fail = [&](crm_status st, const std::string& msg) {
         g_create_error = msg;
@@ -2022,8 +2084,10 @@ crm_status crm_create(const crm_config* cfg, const crm_instance* instances, uint
     if (hipMalloc((void**)&ctx->d_ip, sizeof(InstParams) * n_instances) != hipSuccess ||
         hipMalloc((void**)&ctx->d_ctrl, sizeof(Control)) != hipSuccess)
         return fail(CRM_DEVICE_ERROR, "hipMalloc failed");
-    if (hipHostMalloc((void**)&ctx->pin, kPinControl + kPinDirect, hipHostMallocDefault) != hipSuccess)
-        return fail(CRM_DEVICE_ERROR, "hipHostMalloc failed");
+    {  // the pool's first block (while nothing runs: 12 us here, 30 in set_agents)
+        PinLease pin(ctx);
+        if (pin.take(sizeof(Control)) != hipSuccess) return fail(CRM_DEVICE_ERROR, "hipHostMalloc failed");
+    }
     e = hipMemcpy(ctx->d_ip, ctx->hparams.data(), sizeof(InstParams) * n_instances, hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail(CRM_DEVICE_ERROR, std::string("hipMemcpy: ") + hipGetErrorString(e));
     *out = ctx;
@@ -2979,8 +3043,6 @@ void crm_destroy(crm_ctx* ctx) {
     free_device(ctx);
     if (ctx->d_ip) (void)hipFree(ctx->d_ip);
     if (ctx->d_ctrl) (void)hipFree(ctx->d_ctrl);
-    if (ctx->pin) (void)hipHostFree(ctx->pin);
-    if (ctx->pin_chunks) (void)hipHostFree(ctx->pin_chunks);
     for (auto e : ctx->pin_ev)
         if (e) (void)hipEventDestroy(e);
     for (int i = 0; i < crm_ctx::kTimingPairs; i++) {
@@ -2988,6 +3050,7 @@ void crm_destroy(crm_ctx* ctx) {
         if (ctx->ev_b[i]) (void)hipEventDestroy(ctx->ev_b[i]);
     }
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    pin_pool_leave();
     delete ctx;
 }
 

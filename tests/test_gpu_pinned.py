@@ -1,0 +1,67 @@
+"""Pinned host memory: calls borrow it from a pool of the process, so that contexts hold
+none of their own, and contexts on threads of their own do not see each other's rows."""
+import threading
+
+import numpy as np
+import pytest
+
+from cellular_raza_amd import CartesianCuboid, InstanceSpec, MechanicsBackend, NewtonDamped, NoInteraction
+
+pytestmark = pytest.mark.gpu
+
+
+def context(n, seed):
+    dom = CartesianCuboid.from_boundaries_and_n_voxels([0.0] * 2, [10.0] * 2, [70, 50])
+    g = MechanicsBackend([InstanceSpec(dom, NoInteraction(), NewtonDamped(1.0, 1.0))], dt=0.01)
+    rng = np.random.default_rng(seed)
+    pos, vel = rng.uniform(1e-9, 10.0, (n, 2)), rng.normal(size=(n, 2))
+    g.set_agents(pos, vel)
+    return g, pos, vel
+
+
+def mapped():
+    """KiB of address space of this process."""
+    with open("/proc/self/status") as f:
+        return next(int(line.split()[1]) for line in f if line.startswith("VmSize"))
+
+
+def test_reads_leave_no_memory_with_the_context():
+    """What large reads of sixteen contexts add to the address space (the runtime's own and
+    the threads' stacks and heaps are there from the first context's) is less than half of
+    a block of 8 MiB for each."""
+    made = [context(140000, k) for k in range(17)]
+    for _ in range(3):
+        made[0][0].get_state()
+    before = mapped()
+    for g, pos, vel in made[1:]:
+        p, v = g.get_state()
+        assert np.array_equal(p, pos) and np.array_equal(v, vel)
+        del p, v
+    grown = mapped() - before
+    for g, _, _ in made:
+        g.close()
+    assert grown < 16 * 4096, grown
+
+
+def test_reads_on_many_threads():
+    """More threads than the pool keeps blocks, in every transfer path."""
+    bad = []
+
+    def work(k):
+        for n in (1, 5000, 20000, 60000, 140000):
+            g, pos, vel = context(n + k, 100 * k + 1)
+            for _ in range(3):
+                p, v = g.get_state()
+                if not (np.array_equal(p, pos) and np.array_equal(v, vel)):
+                    bad.append((k, n))
+            g.close()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    g, pos, vel = context(50000, 7)  # after the last context's end the pool begins anew
+    assert np.array_equal(g.get_state()[0], pos)
+    g.close()
