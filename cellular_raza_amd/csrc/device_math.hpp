@@ -173,9 +173,14 @@ __device__ __forceinline__ void direction(const double* z, const RootInv& q, dou
 }
 
 // a / c for a parameter c with its reciprocal from the host (NaN where c is no
-// parameter for `quotient`); r in root_inv's fast range.
+// parameter for `quotient`); a is a distance in root_inv's fast range.
 __device__ __forceinline__ double over(double a, double c, double inv_c, bool fast) {
     return fast && inv_c == inv_c ? quotient(a, c, inv_c) : a / c;
+}
+
+// The same for any a: 0, infinite, NaN, or where the remainder would under- or overflow.
+__device__ __forceinline__ double any_over(double a, double c, double inv_c) {
+    return over(a, c, inv_c, fabs(a) >= 0x1p-900 && fabs(a) <= 0x1p900);
 }
 
 // calculate_morse_interaction, interaction.rs:151-182
@@ -461,7 +466,7 @@ __device__ __forceinline__ void sorting_langevin(const T* z, T attraction, const
             s = (pull / P.cutoff) * __expf(-(sm1 * sm1));
         } else {
             const T sm1 = over(r, R, P.inv_two_radius, root.fast) - T(1);
-            s = over(pull, P.cutoff, P.inv_cutoff, root.fast) * exp(T(-1) * (sm1 * sm1));
+            s = any_over(pull, P.cutoff, P.inv_cutoff) * exp(T(-1) * (sm1 * sm1));
         }
     } else {
 #pragma unroll
