@@ -112,9 +112,13 @@ __device__ __forceinline__ void morse_fast(const float* z, float two_radius, flo
 // root is Goldschmidt's iteration from v_rsq_f64 with two Newton corrections on the
 // exact residual d2 - g^2, the reciprocal follows from its half inverse by one more
 // residual step, and a quotient z / r is Markstein's z * inv corrected by the exact
-// remainder z - q r: each is the correctly rounded value, as sqrt() and / give it,
-// in 3 operations per quotient where an IEEE division takes 12 (4 of them at a
-// quarter of the rate), and 11 for the root and the reciprocal together: the FP64
+// remainder z - q r: roots and quotients are the correctly rounded values, as sqrt() and
+// / give them, in 3 operations per quotient where an IEEE division takes 12 (4 of them at
+// a quarter of the rate), and 15 for the root (10) and the reciprocal (5).  The
+// reciprocal of an r whose significand is all ones is one unit short (the root and the
+// quotients by it are not: 20 million random r and 1.8 million next to powers of two, on
+// the CPU with a v_rsq_f64 off by up to 2^-26); a component z below 2^-968 may be off by
+// its last, subnormal place, as its remainder is.  The FP64
 // force kernels are bound by VALU issue, and the 4M-agent Mie lattice's went from 630
 // to 516 us with bitwise the same forces (with the pow() path in its own kernels,
 // which took 48 spilled registers out of this one; with both in one kernel it ran

@@ -15,7 +15,7 @@
 //                       cells.extend(new_cells)); RodMechanics::divide for mothers
 //   k_grow_start        voxel starts of the grown order (division steps)
 //   k_reflect_key_rod   per-vertex reflection, centroid voxel
-//   (k_rank_ahead and the counting sort of the plain step, then k_advance_step)
+//   (k_rank_ahead and the counting sort of the set-ups, then k_advance_step)
 // Each rod keeps the step of its first history push (`birth`): a daughter starts
 // with an empty AuxStorage, its ring fills from the step after its division.
 #pragma once

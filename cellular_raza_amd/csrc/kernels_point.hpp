@@ -222,9 +222,10 @@ struct Walk3 {
 // Staged records in LDS, addressed by the byte offset kBytes * index: int4 (mixed), or
 // one array of doubles per axis (FP64; the species are bytes beside them).  The
 // capacities keep the occupancy the registers allow: 5 workgroups of at most 32000 bytes
-// per CU (mixed; LDS is given out in 1280-byte granules, and 32512 bytes cost the// fifth), 4 of at most 40960 (FP64).  The FP64 records were double4 (896 of
-// them) and the mixed ones 1024: LDS bounded the tiles, whose own agents filled 64 %
-// of the lanes on the 4M-agent lattice (now 84 %).
+// per CU (mixed; LDS is given out in 1280-byte granules, and 32512 bytes cost the fifth),
+// 4 of at most 40960 (FP64).  The FP64 records were double4 (896 of them) and the mixed
+// ones 1024: LDS bounded the tiles, whose own agents filled 64 % of the lanes on the
+// 4M-agent lattice (now 84 %).
 template <int D, bool MIXED>
 struct LdsRecords;
 template <int D>
@@ -813,7 +814,12 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t& t
 // 1.71 -> 1.33 ms, 100 of 300,000 in FP64 8.10 -> 7.36, 25 of 1600 crowded cells 1.14 ->
 // 0.93, 50 of 12,347 rods 5.50 -> 5.27.  The gather itself got slower, since its stores, not
 // its loads, are now the unaligned side (1M agents 57 -> 65 us, 4M 201 -> 227); other
-// workgroup orders and plain stores changed nothing.
+// workgroup orders and plain stores changed nothing.  Those systems move about one agent in a
+// hundred per step.  Where most agents change voxel in every step, the lists and the scattered
+// stores still cost less than the ranks did in voxels of several agents (free agents, a voxel
+// per step: 1M in voxels of 5 344 -> 301 us a step, of 13 685 -> 359, 300,000 in voxels of
+// 30 458 -> 265, 20,000 in voxels of 500 309 -> 154) and up to 6 % more with one agent per
+// voxel (1M: 247 -> 264; at 0.3 of a voxel per step 172 -> 176).
 // ---------------------------------------------------------------------------
 constexpr int kScanItems = 8;
 constexpr int kScanTileLog2 = 11;
@@ -1627,7 +1633,7 @@ __global__ __launch_bounds__(kBlock) void k_initial_key(Arrays A, StateBuf S, ui
 // Counting sort by voxel (set-up sorts).
 // ---------------------------------------------------------------------------
 // Each thread scans kScanItems consecutive voxels of count + stay into their
-// offsets inside the scan tile (start_local) and clears count for the next step's
+// offsets inside the scan tile (start_local) and clears count for the next sort's
 // ranks; whole groups move as two 16-byte loads per array and two 16-byte stores
 // (count, stay and start_local are 256-byte aligned and a group starts at a
 // multiple of 8 voxels).  bsum[tile] = the tile's sum.

@@ -4,13 +4,16 @@
 // binned by its vertex centroid (bacterial_rods.rs:354-373,536-555).  One lane
 // handles one (rod, vertex); the lanes of a rod are consecutive in a workgroup.
 // Step as launched by the runtime:
-//   k_force_rod              RodInteraction (bacterial_rods.rs:292-336) with the chili
-//                            pair weights (update_mechanics.rs:178-220)
-//   k_key_rod                next vertex positions, per-vertex reflection
-//                            (bacterial_rods.rs:489-533), centroid voxel + rank
-//   k_scan_local/tiles, k_scatter   as for point agents (slots are rods)
-//   k_gather_integrate_rod   RodMechanics::calculate_increment (bacterial_rods.rs:157-240)
-//                            + solver, written into the rod's new slot
+//   k_force_rod    RodInteraction (bacterial_rods.rs:292-336) with the chili pair weights
+//                  (update_mechanics.rs:178-220); its first workgroups then scan the next
+//                  order's voxel counts (scan_moves)
+//   k_gather_rod   RodMechanics::calculate_increment (bacterial_rods.rs:157-240), solver and
+//                  per-vertex reflection (bacterial_rods.rs:489-533), written into the rod's
+//                  slot in the next order; the voxel of its centroid a step later (note_move)
+// With a caller's noise buffer that voxel comes from k_key_rod, and the scan from
+// k_scan_moves, between the two.  Set-up sorts, and every step of the rods' cycle, are the
+// counting sort of point agents (ranks, scan, k_scatter, k_fixup) and k_gather_rod without
+// the update.
 // State arrays are the point arrays with K = nv * dim components per slot; the
 // force kernel reads rods from an AoS copy (rec_rod[slot][K]) written by the gathers.
 #pragma once
