@@ -832,14 +832,15 @@ struct PinLease {
     explicit PinLease(const crm_ctx* ctx) : stream(ctx->stream) {}
     PinLease(const PinLease&) = delete;
     PinLease& operator=(const PinLease&) = delete;
-    hipError_t take(size_t bytes) {
+    bool take_idle(size_t bytes) {  // allocates nothing
         while (kPinBytes[size] < bytes) size++;
-        {
-            std::lock_guard<std::mutex> lock(g_pins.m);
-            for (auto& q : g_pins.idle[size])
-                if (q && !p) std::swap(p, q);
-        }
-        return p ? hipSuccess : hipHostMalloc((void**)&p, kPinBytes[size], hipHostMallocPortable);
+        std::lock_guard<std::mutex> lock(g_pins.m);
+        for (auto& q : g_pins.idle[size])
+            if (q && !p) std::swap(p, q);
+        return p != nullptr;
+    }
+    hipError_t take(size_t bytes) {
+        return take_idle(bytes) ? hipSuccess : hipHostMalloc((void**)&p, kPinBytes[size], hipHostMallocPortable);
     }
     ~PinLease() {
         if (!p) return;
@@ -869,10 +870,15 @@ void pin_pool_leave() {
 }
 
 // The control block after everything queued so far: a one-thread kernel writes it
-// to pinned memory (launch and wait 11 us; a copy to pageable memory 24).
+// to pinned memory (launch and wait 11 us; a copy to pageable memory, for a call that
+// finds every small block in use and may not allocate one, 24).
 crm_status read_control(crm_ctx* ctx, Control& c) {
     PinLease pin(ctx);
-    CRM_HIP(pin.take(sizeof(Control)));
+    if (!pin.take_idle(sizeof(Control))) {
+        CRM_HIP(hipMemcpyAsync(&c, ctx->d_ctrl, sizeof(Control), hipMemcpyDeviceToHost, ctx->stream));
+        CRM_HIP(hipStreamSynchronize(ctx->stream));
+        return CRM_OK;
+    }
     hipLaunchKernelGGL(k_publish_control, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ctrl,
                        reinterpret_cast<Control*>(pin.p));
     CRM_HIP(hipGetLastError());

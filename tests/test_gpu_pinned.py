@@ -5,7 +5,7 @@ import threading
 import numpy as np
 import pytest
 
-from cellular_raza_amd import CartesianCuboid, InstanceSpec, MechanicsBackend, NewtonDamped, NoInteraction
+from cellular_raza_amd import CartesianCuboid, InstanceSpec, MechanicsBackend, NewtonDamped, NoInteraction, SimulationError
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +65,40 @@ def test_reads_on_many_threads():
     g, pos, vel = context(50000, 7)  # after the last context's end the pool begins anew
     assert np.array_equal(g.get_state()[0], pos)
     g.close()
+
+
+def test_steps_and_errors_on_many_threads():
+    """Every step reads the control block: more threads than the pool keeps blocks, one of
+    them with an agent that leaves the domain."""
+    bad = []
+
+    def work(k):
+        dom = CartesianCuboid.from_boundaries_and_n_voxels([0.0] * 2, [10.0] * 2, [7, 5])
+        g = MechanicsBackend([InstanceSpec(dom, NoInteraction(), NewtonDamped(-5.0 if k == 3 else 0.0, 1.0))], dt=0.1,
+                             mechanics_solver_order=0)
+        pos, vel = np.full((300, 2), 5.0), np.zeros((300, 2))
+        vel[7, 0] = 5.0 if k == 3 else 0.01 * (k + 1)
+        g.set_agents(pos, vel)
+        done = 0
+        try:
+            for done in range(60):
+                g.step(1)
+        except SimulationError as e:
+            if k != 3 or e.kind != "BoundaryError":
+                bad.append((k, done, str(e)))
+            failed.append(done)
+        if k != 3:
+            want = 5.0
+            for _ in range(60):
+                want = want + 0.1 * (0.01 * (k + 1))
+            if g.info().step != 60 or g.get_positions()[7, 0] != want:
+                bad.append((k, done, g.get_positions()[7, 0], want))
+        g.close()
+
+    failed = []
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad and len(failed) == 1, (bad, failed)
