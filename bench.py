@@ -551,7 +551,7 @@ def main():
         achieved_tflops = flops_agent * N / (t_force_ms * 1e-3) / 1e12
     traffic = profile_figure("hbm_bytes_per_dispatch", force_kernel, args.workload)
     step_bytes = None
-    if nv == 1:  # the step's byte model: force + integrator + counting sort (points)
+    if nv == 1:  # byte model of a step (points): force + integrator + a counting sort that moves the state again
         langevin = wl.noise == "philox"
         force_w = 4 * D if has_mixed else 8 * D
         b_i = (8 * D + 8 * D + force_w + 32 * D + (8 * D if langevin else 0)) + (8 * D + 8 * D + 16 * D + 4)
