@@ -171,8 +171,9 @@ enum { kNumKernelClasses = CRM_KERNEL_COUNT };
 // call borrows (PinLease).  Read-backs up to kPinDirect are written there by the gathering
 // kernel itself and moved on in parts of kPinPart bytes by a host thread for every whole
 // kPinPerThread of them; larger ones are copied out through kPinWorkers chunks of kPinChunk
-// bytes, each queued, awaited and emptied by a host thread of its own: one thread fills fresh pages of the caller's array at 4.5 GB/s (page faults), two
-// at 8, four at 12.5, eight at 19-20 GB/s (48 MB and 192 MB; the link carries 55 GB/s).
+// bytes, each queued, awaited and emptied by a host thread of its own: one thread fills
+// fresh pages of the caller's array at 4.5 GB/s (page faults), two at 8, four at 12.5, eight
+// at 19-20 GB/s (48 MB and 192 MB; the link carries 55 GB/s).
 // The lines lie where both sides meet: threads that call HIP cost 20 us more than ones
 // that copy (get_state of 516 KB 98 us with two of them, 52 with the kernel's own stores
 // and none), a second thread pays from 1 MB on (0.5 MB to a thread: forces of 90,000
